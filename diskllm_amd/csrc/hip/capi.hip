@@ -198,7 +198,7 @@ dlk::RowParams rows_from(const dlk::RowParams &p, int r0) {
 int launch_topk(dlk::RowParams &p, int rows, int vocab, hipStream_t stream) {
     using namespace dlk;
     const int T = kTopkThreads;
-    if (((uintptr_t)p.logits & 15) != 0 || (p.ld & 3) != 0) return 1;
+    if (((uintptr_t)p.logits & 3) != 0) return 1;     /* (rows of any stride: load4) */
     const int k = p.greedy ? 1 : p.top_k;
     if (k > kTopkMaxK) return 1;
     if (p.plan.hcap > kTopkHcapMax) return 1;     /* (the host stages longer histories elsewhere) */
@@ -284,8 +284,8 @@ int launch_full(dlk::RowParams &p, int rows, int vocab, int force_exact, int no_
     if (p.minp_on && p.topp_on && p.top_p <= 0.0f) return 1;
     if (!(p.inv_temp < INFINITY)) return 1;            /* (v - M) * inv_t is NaN at the maximum */
     if (p.plan.hcap > 2 * T) return 1;                 /* one or two history ids per thread, loaded first */
-    if (((uintptr_t)p.logits & 15) != 0 || (p.ld & 3) != 0) return 1;
-    if (vocab < 8192 || (vocab & 3) != 0) return 1;   /* whole 16-byte groups per row */
+    if (((uintptr_t)p.logits & 3) != 0) return 1;      /* (rows of any stride and length: load4) */
+    if (vocab < 8192) return 1;                        /* not one workgroup's slice */
     /* about 512 workgroups: two per CU on 256 CUs */
     int G = (512 + rows - 1) / rows;
     if (G > kFullMaxG) G = kFullMaxG;

@@ -24,6 +24,15 @@ DLK_DEV float u2f(uint32_t u) { return __uint_as_float(u); }
 DLK_DEV uint64_t d2u(double d) { return (uint64_t)__double_as_longlong(d); }
 DLK_DEV double u2d(uint64_t u) { return __longlong_as_double((long long)u); }
 
+/* Four consecutive floats from any float address.  A global 16-byte load needs only
+ * 4-byte alignment on gfx950, so rows of any stride take the same instruction as
+ * aligned ones (a wave's 1 KB may touch one cache line more). */
+typedef float f4_any __attribute__((ext_vector_type(4), aligned(4)));
+DLK_DEV float4 load4(const float *p) {
+    const f4_any x = *(const f4_any *)p;
+    return make_float4(x.x, x.y, x.z, x.w);
+}
+
 DLK_DEV uint64_t ballot(bool p) { return __ballot(p); }
 DLK_DEV int first_lane(uint64_t m) { return m ? __builtin_ctzll(m) : 64; }
 

@@ -52,15 +52,16 @@ DLK_DEV uint64_t at_ld64(const uint64_t *a) {
 
 
 
-/* Issues the loads of a slice: 16-byte groups of logits (an out-of-range group
- * reads the slice start instead) and, with a mask, each group's mask word. */
+/* Issues the loads of a slice: groups of four logits (one that reaches past the
+ * slice reads its last four instead; the row has at least four elements) and,
+ * with a mask, each group's mask word. */
 template <int EPT, int J0, int J1>
 __device__ __forceinline__ void load_slice(const float *lg, const uint32_t *mk, int s0, int s1, int t, int T,
                                            float4 *raw, uint32_t *mwd) {
 #pragma unroll
     for (int j4 = J0; j4 < J1; j4++) {
         const int i0 = s0 + 4 * (t + j4 * T);
-        raw[j4] = *(const float4 *)(lg + (i0 < s1 ? i0 : s0));
+        raw[j4] = load4(lg + min(i0, s1 - 4));
         mwd[j4] = (mk && i0 < s1) ? mk[i0 >> 5] : 0xffffffffu;
     }
 }
@@ -410,7 +411,14 @@ __device__ __forceinline__ void draw_fix(const FullParams &f, int row, int h, ui
 #pragma unroll
         for (int k = 0; k < 2; k++) {
             const int i0 = s0 + 4 * (t + (jb + k) * T);
-            raw[k] = i0 < s1 ? *(const float4 *)(lg + i0) : make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
+            raw[k] = make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
+            if (i0 + 3 < s1) {
+                raw[k] = load4(lg + i0);
+            } else if (i0 < s1) {              /* the row's last group, of one to three elements */
+                raw[k].x = lg[i0];
+                if (i0 + 1 < s1) raw[k].y = lg[i0 + 1];
+                if (i0 + 2 < s1) raw[k].z = lg[i0 + 2];
+            }
         }
 #pragma unroll
         for (int k = 0; k < 2; k++) {
@@ -621,6 +629,23 @@ __global__ __launch_bounds__(kFullThreads) void full_kernel(FullParams f) {
             atomicAdd(&hcnt[h], 1u);
         }
     }
+    /* a row that is no whole number of groups: the four ids of its last group
+     * (some past the row: -inf) are patched too, whether the history holds them
+     * or not, so the loads and the merge stay whole groups (hslots is at least
+     * 2 * hcap >= hcap + 64, so they have room) */
+    const int tail0 = V & ~3;
+    const bool tail = (V & 3) != 0 && tail0 >= s0 && tail0 < s1;
+    int tslot = -1;
+    if (DLK_COLD(tail) && t < 4) {
+        const int id = tail0 + t;
+        uint32_t h = ((uint32_t)id * 0x9E3779B1u) >> hshift;
+        for (int probe = 0; probe < hslots; probe++) {
+            const int old = atomicCAS(&hkey[h], -1, id);
+            if (old == -1) { tslot = (int)h; atomicOr(&sbits[(id - s0) >> 5], 1u << ((id - s0) & 31)); }
+            if (old == -1 || old == id) break;
+            h = (h + 1) & (uint32_t)(hslots - 1);
+        }
+    }
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < HP; k++) {
@@ -630,6 +655,17 @@ __global__ __launch_bounds__(kFullThreads) void full_kernel(FullParams f) {
             if (!((gm[k] >> (hid[k] & 31)) & 1u)) x = -INFINITY;
             hcnt[oslot[k]] = __float_as_uint(penalize(x, (int)hcnt[oslot[k]], p));
         }
+    }
+    if (DLK_COLD(tslot >= 0)) {
+        const int id = tail0 + t, cnt = (int)hcnt[tslot];
+        float x = -INFINITY;
+        if (id < V) {
+            x = lg[id];
+            if (CAP) x = dlk_softcap_glibc(x, p.cap);
+            if (mk && !((mk[id >> 5] >> (id & 31)) & 1u)) x = -INFINITY;
+            if (cnt > 0) x = penalize(x, cnt, p);
+        }
+        hcnt[tslot] = __float_as_uint(x);
     }
     /* the patch of a marked id */
     auto hpatch = [&](int id) {
@@ -641,8 +677,8 @@ __global__ __launch_bounds__(kFullThreads) void full_kernel(FullParams f) {
     const float r = rand_f32_from(st);
     __syncthreads();
 
-    /* masked entries -inf, patched entries their penalised value; the row is a
-     * whole number of 4-element groups (the host routes other rows elsewhere) */
+    /* masked entries -inf, patched entries their penalised value (and those of
+     * the row's last group, where it is not whole) */
     float v[EPT];
     float tm = -INFINITY;
     bool bad = false;                              /* NaN or +inf after penalties */

@@ -87,9 +87,9 @@ DLK_DEV float live_or_ninf(float x, uint32_t live, int c) {
     return __int_as_float((__float_as_int(x) & m) | ((int)0xff800000 & ~m));
 }
 
-/* The 16-byte group of row elements i0 .. i0 + 3 (i0 a multiple of 4), -inf past s1. */
+/* The group of row elements i0 .. i0 + 3 (i0 a multiple of 4), -inf past s1. */
 DLK_DEV float4 load_group(const float *lg, int i0, int s1) {
-    if (i0 + 3 < s1) return *(const float4 *)(lg + i0);
+    if (i0 + 3 < s1) return load4(lg + i0);
     float4 x = make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
     if (i0 < s1) x.x = lg[i0];
     if (i0 + 1 < s1) x.y = lg[i0 + 1];
@@ -231,7 +231,7 @@ __global__ __launch_bounds__(kTopkThreads, 8) void topk_kernel(TopkParams f) {
     auto load_batch = [&](float4 (&x)[4], uint32_t (&m)[4], int b) {
         if (gpos(b, 0) - 4 * t + 16 * T <= s1) {
 #pragma unroll
-            for (int j = 0; j < 4; j++) x[j] = *(const float4 *)(lg + gpos(b, j));
+            for (int j = 0; j < 4; j++) x[j] = load4(lg + gpos(b, j));
 #pragma unroll
             for (int j = 0; j < 4; j++) m[j] = mk ? mk[gpos(b, j) >> 5] : 0xffffffffu;
         } else {
