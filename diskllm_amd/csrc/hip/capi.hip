@@ -222,7 +222,7 @@ int launch_topk(dlk::RowParams &p, int rows, int vocab, hipStream_t stream) {
         const size_t fall_b = (size_t)p.plan.kp * 8 + 2048 * 4;
         size_t work = slice_b > merge_b ? slice_b : merge_b;
         if (fall_b > work) work = fall_b;
-        return fixed_lds(p.plan) + r16(64 * 4) + r16((size_t)kSelWords * 4) + r16((size_t)(3 * G + 2) * 4) + work;
+        return fixed_lds(p.plan) + r16(64 * 4) + r16((size_t)kSelWords * 4) + r16((size_t)(4 * G + 2) * 4) + work;
     };
     /* the most workgroups per row that still run as one resident round (each
      * workgroup's post-stream latency is then paid once), else the fewest */
@@ -250,7 +250,10 @@ int launch_topk(dlk::RowParams &p, int rows, int vocab, hipStream_t stream) {
     int S = slice_of(gmin);
     for (int g = gmax; g >= gmin; g--) {
         const int s = slice_of(g), gr = (vocab + s - 1) / s;
-        if ((int64_t)rows * gr <= resident(lds_for(s, gr))) { S = s; break; }
+        /* (greedy: eight one-batch slices on a CU cost more in their tails than four
+         * of two batches: 64 x 128,256 took 20.3 us against 15.5) */
+        const int64_t fit = resident(lds_for(s, gr)) / (p.greedy && s < 2 * unit ? 2 : 1);
+        if ((int64_t)rows * gr <= fit) { S = s; break; }
     }
     const int G = (vocab + S - 1) / S;
     TopkParams f;

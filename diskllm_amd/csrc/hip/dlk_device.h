@@ -166,6 +166,13 @@ DLK_DEV uint32_t wave_minmax_u32(uint32_t v) {
     o = (uint32_t)__builtin_amdgcn_update_dpp(id, (int)v, kDppRowBcast31, 0xc, 0xf, false); v = MIN ? min(v, o) : max(v, o);
     return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
 }
+/* Sum over the 64 lanes (every lane gets it). */
+DLK_DEV int wave_sum_i32(int v) {
+    uint32_t x = row_scan_u32((uint32_t)v);
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, kDppRowBcast15, 0xa, 0xf, false);
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, kDppRowBcast31, 0xc, 0xf, false);
+    return __builtin_amdgcn_readlane((int)x, 63);
+}
 /* Inclusive wave prefix with saturation at `cap` (values <= cap). */
 DLK_DEV uint32_t wave_scan_sat_u32(uint32_t x, uint32_t cap) {
     uint32_t t;

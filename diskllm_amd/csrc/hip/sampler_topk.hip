@@ -64,14 +64,15 @@ DLK_DEV float penalised(const RowParams &p, float x, int cnt) {
  * their LDS list.  Ties that the cap creates are resolved by the order
  * (y desc, index asc) of the collected candidates and the merge's certificate. */
 
-/* Key of the r-th largest of the 128 ascending keys a, b held two per lane: the
- * largest K with at least r keys >= K, found bit by bit from ballots (no LDS, no
- * barrier).  Every lane returns it. */
+/* A bound just below the r-th largest of the 128 ascending keys a, b held two per
+ * lane: the largest K of 20 significant bits with at least r keys >= K, found bit
+ * by bit from ballots (no LDS, no barrier; a rolled loop, since straight code that
+ * runs once per launch is paid in instruction-cache misses).  Every lane returns it. */
 DLK_DEV uint32_t wave_rth_key(uint32_t a, uint32_t b, int r) {
     uint32_t K = 0;
-#pragma unroll
-    for (int bit = 31; bit >= 0; bit--) {
-        const uint32_t c = K | (1u << bit);
+#pragma unroll 1
+    for (uint32_t bit = 0x80000000u; bit >= 0x1000u; bit >>= 1) {
+        const uint32_t c = K | bit;
         const int n = __popcll(ballot(a >= c)) + __popcll(ballot(b >= c));
         if (n >= r) K = c;
     }
@@ -87,10 +88,12 @@ DLK_DEV float live_or_ninf(float x, uint32_t live, int c) {
     return __int_as_float((__float_as_int(x) & m) | ((int)0xff800000 & ~m));
 }
 
-/* The group of row elements i0 .. i0 + 3 (i0 a multiple of 4), -inf past s1. */
+/* The group of row elements i0 .. i0 + 3 (i0 a multiple of 4); 0 past s1 (no caller
+ * takes an entry past s1 for live; a -inf there would look like a non-finite
+ * logit and send every short last slice through the exact pass, 3 to 6 us). */
 DLK_DEV float4 load_group(const float *lg, int i0, int s1) {
     if (i0 + 3 < s1) return load4(lg + i0);
-    float4 x = make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
+    float4 x = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     if (i0 < s1) x.x = lg[i0];
     if (i0 + 1 < s1) x.y = lg[i0 + 1];
     if (i0 + 2 < s1) x.z = lg[i0 + 2];
@@ -211,7 +214,7 @@ __global__ __launch_bounds__(kTopkThreads, 8) void topk_kernel(TopkParams f) {
     unsigned char *q = L.region;
     int *misc = (int *)carve(q, 64 * 4);
     int *selh = (int *)carve(q, kSelWords * 4);                           /* radix-select histogram */
-    uint32_t *sk = (uint32_t *)carve(q, (size_t)(3 * G + 2) * 4);          /* merge: per-slice words, tau */
+    uint32_t *sk = (uint32_t *)carve(q, (size_t)(4 * G + 2) * 4);          /* merge: per-slice words, tau, ck */
     unsigned char *work = q;
     uint32_t *gbits = (uint32_t *)carve(q, (size_t)(f.S / 128) * 4);       /* slice: groups holding penalised ids */
     uint32_t *grp = (uint32_t *)carve(q, (size_t)f.grp_cap * 4);           /* slice: listed groups */
@@ -271,6 +274,11 @@ __global__ __launch_bounds__(kTopkThreads, 8) void topk_kernel(TopkParams f) {
     }
     for (int i = t; i < f.S / 128; i += T) gbits[i] = 0;
     if (t < 16) misc[t] = 0;                       /* (16.. are written before they are read) */
+    int *hkey = (int *)L.hsort;                    /* the history's hash table (below), cleared while batch 0 lands */
+    int *hcnt = (int *)L.pval;
+    const int hslots = 2 * p.plan.hcap;            /* a power of two */
+    if (nh > 0)
+        for (int i = t; i < hslots; i += T) { hkey[i] = -1; hcnt[i] = 0; }
 
     /* penalty patches of the ids inside this slice: misc[0] entries of
      * (pid, pval), their groups' bits in gbits, misc[11] of them allowed by the
@@ -282,15 +290,8 @@ __global__ __launch_bounds__(kTopkThreads, 8) void topk_kernel(TopkParams f) {
      * Keys span hsort and pid, counts pval and pcnt (carved back to back, each
      * hcap words, a multiple of 16 bytes); pid and pval are reused for the
      * patch list only after the counts have been read. */
-    int *hkey = (int *)L.hsort;
-    int *hcnt = (int *)L.pval;
-    const int hslots = 2 * p.plan.hcap;            /* a power of two */
     const int hshift = 32 - (31 - __clz(hslots));
     constexpr int kPer = kTopkHcapMax / kTopkThreads;   /* history entries per thread (nh <= hcap) */
-    auto stage_history = [&]() {
-        for (int i = t; i < hslots; i += T) { hkey[i] = -1; hcnt[i] = 0; }
-        __syncthreads();
-    };
     auto count_patches = [&]() {
         int oslot[kPer], oid[kPer];
         float ov[kPer];
@@ -346,14 +347,14 @@ __global__ __launch_bounds__(kTopkThreads, 8) void topk_kernel(TopkParams f) {
         __syncthreads();
     };
     if (GREEDY) {                                  /* greedy streams exact values */
-        stage_history();
-        count_patches();
+        __syncthreads();
+        if (nh > 0) count_patches();
     }
     int np = GREEDY ? min(misc[0], p.plan.hcap) : 0;
 
     /* ---- 2. stream the slice -------------------------------------------- */
     float m1 = -INFINITY, m2 = -INFINITY;          /* the lane's two best group maxima */
-    int gi = -1;                                   /* GREEDY: first group holding m1 */
+    int gi = -1;                                   /* GREEDY: first index holding m1 */
     int nfl = 0;                                   /* stream entries allowed by the mask */
     uint64_t spc = 0;                              /* ballot: a non-finite raw logit seen */
     float thr = -INFINITY;
@@ -378,7 +379,9 @@ __global__ __launch_bounds__(kTopkThreads, 8) void topk_kernel(TopkParams f) {
             }
             gm[j] = fmaxf(fmaxf(e[0], e[1]), fmaxf(e[2], e[3]));
             if (GREEDY) {
-                if (gm[j] > m1) { m1 = gm[j]; gi = i0; }
+                /* (the first entry of the group that holds its maximum) */
+                const int c = e[0] == gm[j] ? 0 : e[1] == gm[j] ? 1 : e[2] == gm[j] ? 2 : 3;
+                if (gm[j] > m1) { m1 = gm[j]; gi = i0 + c; }
             } else {
                 nfl += __popc(live);
                 m2 = fmaxf(m2, fminf(m1, gm[j]));
@@ -436,15 +439,9 @@ __global__ __launch_bounds__(kTopkThreads, 8) void topk_kernel(TopkParams f) {
     int bi = 0x7fffffff, nf = 0, irr = 0, kept = 0, complete = 1;
     uint32_t last_key = 0, fnan = 0;
     if (GREEDY) {
-        /* ---- 3g. slice maximum and its lowest index --------------------- */
-        if (gi >= 0) {
-            const float4 v = load_group(lg, gi, s1);
-            const uint32_t mwg = mk ? mk[gi >> 5] >> (gi & 31) : 0xFu;
-            const uint32_t live = group_live(mwg, gbits, L.pid, np, gi, s0, s1);
-            const float e[4] = {v.x, v.y, v.z, v.w};
-            for (int c = 3; c >= 0; c--)
-                if (live_or_ninf(e[c], live, c) == m1) bi = gi + c;
-        }
+        /* ---- 3g. slice maximum and its lowest index (kept by the stream: every
+         *      lane's best group read again cost the last blocks 6 us) ------- */
+        if (gi >= 0) bi = gi;
         bm = m1;
         for (int k2 = t; k2 < np; k2 += T) {
             const float y = L.pval[k2];
@@ -463,20 +460,20 @@ __global__ __launch_bounds__(kTopkThreads, 8) void topk_kernel(TopkParams f) {
         }
     } else {
         /* ---- 3. patches, finite count; an exact pass when needed -------- */
-        {
-            /* the final threshold, from every batch (read after the patches' barriers) */
+        if (nb & (nb - 1)) {
+            /* the final threshold, from every batch (read after the patches'
+             * barriers; a power of two of batches took it after the last one) */
             const uint32_t K = wave_rth_key(asc_key(m1), asc_key(m2), (f.KP + 3) / 4);
             if (lane == 0) misc[16 + w] = (int)K;
         }
-        int wn = nfl;
-        for (int m = 32; m >= 1; m >>= 1) wn += shfl_xor(wn, m);
+        const int wn = wave_sum_i32(nfl);
         if (lane == 0) {
             atomicAdd(&misc[3], wn);
             if (spc) misc[8] = 1;
         }
-        stage_history();
-        count_patches();
-        np = min(misc[0], p.plan.hcap);
+        /* (the table was cleared before the stream's first barrier) */
+        if (nh > 0) count_patches();
+        np = nh > 0 ? min(misc[0], p.plan.hcap) : 0;
         float pmax = -INFINITY;
         int pn = 0, pirr = 0;
         for (int k2 = t; k2 < np; k2 += T) {       /* the patches: capped values under CAP */
@@ -614,8 +611,9 @@ __global__ __launch_bounds__(kTopkThreads, 8) void topk_kernel(TopkParams f) {
                 __syncthreads();
             }
             int n = C;
-            /* only the KP best are sorted (KP, plus any ties at the KP-th key) */
-            if (n > f.KP + 16 && n <= T) n = keep_best(cbuf, n, f.KP, &misc[20]);
+            /* of many, only the KP best are sorted (KP, plus any ties at the KP-th
+             * key); up to half the block the sort is cheaper than the selection */
+            if (n > max(f.KP, T / 2) && n <= T) n = keep_best(cbuf, n, f.KP, &misc[20]);
             if (n <= T) {
                 rank_sort_distinct(cbuf, n);
             } else {
@@ -683,8 +681,8 @@ __global__ __launch_bounds__(kTopkThreads, 8) void topk_kernel(TopkParams f) {
         sw[128 + t] = nfin_h;
         sw[192 + t] = nan_h;
     }
-    uint32_t *tau = sk + 3 * G, *tau2 = sk + 3 * G + 1;
-    if (t == 0) { pub32(&f.counters[row], 0u); *tau = 0xffffffffu; *tau2 = 0u; misc[46] = 0; }
+    uint32_t *tau = sk + 3 * G, *ck = tau + 2;    /* ck: the lists' c-th keys */
+    if (t == 0) { pub32(&f.counters[row], 0u); *tau = 0xffffffffu; misc[46] = 0; }
     __syncthreads();
     /* every wave reduces the slices itself (the argmax keeps the larger value,
      * ties to the lower index, as in order) */
@@ -699,16 +697,20 @@ __global__ __launch_bounds__(kTopkThreads, 8) void topk_kernel(TopkParams f) {
         total = (int)sk[3 * lane];
         overflow = (int)sk[3 * lane + 1] == -1;
     }
-    for (int m2 = 32; m2 >= 1; m2 >>= 1) {
-        const float om = shfl_xor(M, m2);
-        const int oa = shfl_xor(amax, m2);
-        if (om > M || (om == M && oa < amax)) { M = om; amax = oa; }
-        NF += shfl_xor(NF, m2);
-        first_nan |= shfl_xor(first_nan, m2);
-        irregular |= shfl_xor(irregular, m2);
-        total += shfl_xor(total, m2);
-        overflow |= shfl_xor(overflow, m2);
+    if (GREEDY) {
+        for (int m2 = 32; m2 >= 1; m2 >>= 1) {
+            const float om = shfl_xor(M, m2);
+            const int oa = shfl_xor(amax, m2);
+            if (om > M || (om == M && oa < amax)) { M = om; amax = oa; }
+        }
+    } else {
+        M = wave_max_dpp(M);                       /* (not used where irregular) */
+        NF = wave_sum_i32(NF);
+        total = wave_sum_i32(total);
+        irregular = ballot(irregular != 0) != 0;
+        overflow = ballot(overflow != 0) != 0;
     }
+    first_nan = ballot(first_nan != 0) != 0;
     const int n_out = p.n_out;
     auto out_cands_empty = [&](float pr, float lpv, bool ids_idx, int kk) {
         for (int j = t; j < n_out; j += T) {
@@ -718,7 +720,7 @@ __global__ __launch_bounds__(kTopkThreads, 8) void topk_kernel(TopkParams f) {
             if (p.out_cand_logprobs) p.out_cand_logprobs[o] = lpv;
         }
     };
-    if (p.greedy) {
+    if (GREEDY) {
         if (t == 0) p.out_ids[row] = (first_nan || amax == 0x7fffffff) ? 0 : amax;
         out_cands_empty(0.0f, -INFINITY, false, 0);
         return;
@@ -752,25 +754,30 @@ __global__ __launch_bounds__(kTopkThreads, 8) void topk_kernel(TopkParams f) {
     if (ok) {
         /* bounds for the sort: list h is in logit order and s is monotone in
          * the logit, so at least k entries have s >= the s of any list's k-th
-         * entry (tau), and when every list holds cq = ceil(k / G) entries, at
-         * least G * cq >= k have s >= the smallest s among the lists' cq-th
-         * entries (tau2); anything whose s is below the better bound is not in
-         * the top k */
-        const int cq = (k + G - 1) / G;
-        const bool all_cq = __popcll(ballot(lane < G && (int)sk[3 * lane] >= cq)) == (unsigned)G;
+         * entry (tau), and with m = ceil(k / c), at least m * c >= k have
+         * s >= the m-th best of the lists' c-th entries; anything whose s is
+         * below the better bound is not in the top k.  c = ceil(k / G) takes
+         * (nearly) the worst list, which a short last slice makes a poor bound:
+         * some 130 to over 600 entries survived at 32 lists and k = 40 (more than
+         * buf_cap sends the row to the whole-row selection, 460 us).
+         * c = floor(k / G) + 2 takes a middle one and leaves about 1.7 k; few
+         * lists (long ones, alike in what they hold) keep the first. */
+        const int cq = G > 8 ? min(k / G + 2, k) : (k + G - 1) / G;
+        const int mq = (k + cq - 1) / cq;
         /* (list h, slot j) of entry i = t + u * T, stepped without a division;
-         * tau and tau2 reduced in the wave first (one LDS atomic per wave) */
+         * tau reduced in the wave first (one LDS atomic per wave) */
         const int qT = T / KP, rT = T - qT * KP;
         int h = t / KP, j = t - h * KP;
-        uint32_t kmin = 0xffffffffu, kmax = 0u;
+        uint32_t kmin = 0xffffffffu;
 #pragma unroll
         for (int u = 0; u < kMergePerThread; u++) {
             const int i = t + u * T;
             if (i < GK && j < (int)sk[3 * h]) {
                 cv[u] = ((uint64_t)desc_key((key_value((uint32_t)(cv[u] >> 32)) - M) * R.inv_t) << 32) |
                         (cv[u] & 0xffffffffull);
-                if (j == k - 1) kmin = min(kmin, (uint32_t)(cv[u] >> 32));
-                if (j == cq - 1) kmax = max(kmax, (uint32_t)(cv[u] >> 32));
+                const uint32_t key = (uint32_t)(cv[u] >> 32);
+                if (j == k - 1) kmin = min(kmin, key);
+                if (j == cq - 1) ck[h] = key;
             } else {
                 cv[u] = ~0ull;
             }
@@ -779,13 +786,19 @@ __global__ __launch_bounds__(kTopkThreads, 8) void topk_kernel(TopkParams f) {
             if (j >= KP) { j -= KP; h++; }
         }
         kmin = wave_minmax_u32<true>(kmin);
-        kmax = wave_minmax_u32<false>(kmax);
-        if (lane == 0) {
-            if (kmin != 0xffffffffu) atomicMin(tau, kmin);
-            if (kmax != 0u) atomicMax(tau2, kmax);
-        }
+        if (lane == 0 && kmin != 0xffffffffu) atomicMin(tau, kmin);
         __syncthreads();
-        const uint32_t tk = all_cq ? min(*tau, *tau2) : *tau;
+        /* the m-th smallest of the lists' keys by its high 16 bits (a list
+         * shorter than c has none); every wave finds it itself */
+        uint32_t tk = *tau;
+        {
+            const uint32_t ka = lane < G && (int)sk[3 * lane] >= cq ? ck[lane] : 0xffffffffu;
+            uint32_t K = 0;
+#pragma unroll 1
+            for (uint32_t bit = 0x80000000u; bit >= 0x10000u; bit >>= 1)
+                if ((int)__popcll(ballot(ka < (K | bit))) < mq) K |= bit;
+            tk = min(tk, K | 0xffffu);
+        }
         /* the survivors to LDS: one reservation per wave */
         uint64_t balu[kMergePerThread];
         int tot = 0;
@@ -796,7 +809,7 @@ __global__ __launch_bounds__(kTopkThreads, 8) void topk_kernel(TopkParams f) {
         }
         int base = 0;
         if (lane == 0 && tot) base = atomicAdd(&misc[46], tot);
-        base = shfl(base, 0);
+        base = __builtin_amdgcn_readfirstlane(base);
 #pragma unroll
         for (int u = 0; u < kMergePerThread; u++) {
             const int at = base + lanes_below(balu[u]);
@@ -808,8 +821,8 @@ __global__ __launch_bounds__(kTopkThreads, 8) void topk_kernel(TopkParams f) {
         if (DLK_COLD(nsort > f.buf_cap)) {
             ok = false;
         } else {
-            /* only the k best are sorted (k, plus any ties at the k-th s-key) */
-            if (nsort > k + 16 && nsort <= T) nsort = keep_best(buf, nsort, k, &misc[48]);
+            /* of many, only the k best are sorted (k, plus any ties at the k-th s-key) */
+            if (nsort > max(k, T / 2) && nsort <= T) nsort = keep_best(buf, nsort, k, &misc[48]);
             if (DLK_HOT(nsort <= T)) {
                 rank_sort_distinct(buf, nsort);
             } else {

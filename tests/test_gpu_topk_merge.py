@@ -1,0 +1,56 @@
+"""The top-k kernel's merge of its slices' lists where its bounds and sorts can go wrong: a short last slice, one
+list, few and many lists, a top k that lies in one slice or in runs of equal logits, lists shorter than the bound
+takes from them, and survivors around the sizes at which the sort shares a key among threads."""
+import numpy as np
+import pytest
+
+from diskllm_amd import workloads as W
+from test_gpu_edges import make, mask_rows, run_and_check
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("V,rows", [(128256, 1), (131072, 2), (4100, 3), (69632, 40), (65537, 700)])
+@pytest.mark.parametrize("k", [1, 8, 40, 64, 100, 250])
+def test_topk_lists(cuda, V, rows, k):
+    rng = np.random.default_rng(V + k)
+    lg = rng.normal(0, 2.5, size=(rows, V)).astype(np.float32)
+    for r in range(rows):
+        kind = r % 5
+        if kind == 1:                                  # the top k in consecutive entries of one slice
+            at = int(rng.integers(0, V - 2 * k))
+            lg[r, at:at + 2 * k] += np.float32(30)
+        elif kind == 2:                                # and in the row's last entries
+            lg[r, V - k - 3:] += np.float32(30)
+        elif kind == 3:                                # runs of equal logits
+            lg[r] = np.round(lg[r] * 2) / 2
+        elif kind == 4:                                # sorted rows: the lists hold very unlike values
+            lg[r] = np.sort(lg[r])[::(-1) ** (r // 5)]
+    hist = [rng.integers(0, V, 30) for _ in range(rows)]
+    w = make(f"lists-{V}-{k}", rows, V, seed=k, logits=lg, temperature=0.8, top_k=k, top_p=0.97, rep=1.3, hist=hist,
+             n_out=min(k, 16))
+    run_and_check(w, 0)
+
+
+@pytest.mark.parametrize("allowed", [3, 60, 400, 3000])
+def test_topk_short_lists(cuda, allowed):
+    """Masks that leave most lists shorter than the bound's c, some empty, in all fewer than k or a little more."""
+    V, rows = 128256, 4
+    rng = np.random.default_rng(allowed)
+    mask = mask_rows(rows, V, [rng.choice(V if r % 2 else V // 3, allowed, replace=False) for r in range(rows)])
+    w = make(f"short-{allowed}", rows, V, seed=allowed, temperature=0.7, top_k=50, top_p=0.95, mask=mask, n_out=8,
+             order=W.ORDER_REFERENCE)
+    run_and_check(w, 0)
+
+
+@pytest.mark.parametrize("rows,V", [(64, 128256), (1, 4097), (3, 70001), (300, 32768)])
+def test_greedy_first_of_equal_maxima(cuda, rows, V):
+    """The lowest index of the maximum, wherever in a group and slice it lies, the maximum penalised or masked too."""
+    rng = np.random.default_rng(rows)
+    lg = rng.normal(0, 2, size=(rows, V)).astype(np.float32)
+    hist = []
+    for r in range(rows):
+        at = rng.choice(V, 4, replace=False)
+        lg[r, at] = np.float32(20)
+        hist.append([int(at.min())] if r % 3 == 0 else [int(rng.integers(0, V))])
+    run_and_check(make(f"greedy-{rows}", rows, V, seed=rows, logits=lg, temperature=0.0, rep=1.5, hist=hist), 0)
