@@ -36,6 +36,7 @@ namespace {
 constexpr size_t kMaxLds = 160 * 1024;
 constexpr int kMaxTopKLds = 4096;          /* larger top-k: candidates in global memory */
 constexpr int kHcapDirect = 1024;          /* longer histories: penalties applied to a scratch copy first */
+constexpr size_t kFullWorkspace = (size_t)512 << 20;      /* workspace per launch of the fused kernel */
 constexpr size_t kGlobalTopkBudget = (size_t)256 << 20;   /* workspace per launch of the large-k row kernel */
 constexpr int kLsdWords = 256 + 16 * 256 + 16;            /* select_top_k_global's LDS words */
 
@@ -289,14 +290,21 @@ int launch_full(dlk::RowParams &p, int rows, int vocab, int force_exact, int no_
     if (p.plan.hcap > 2 * T) return 1;                 /* one or two history ids per thread, loaded first */
     if (((uintptr_t)p.logits & 3) != 0) return 1;      /* (rows of any stride and length: load4) */
     if (vocab < 8192) return 1;                        /* not one workgroup's slice */
-    /* about 512 workgroups: two per CU on 256 CUs */
+    /* about 512 workgroups, two per CU on 256 CUs, and no more than 40 entries
+     * per thread where the row's workgroups allow: 48 take the kernel past 128
+     * VGPRs, one workgroup per CU (512 x 151,936: 670 us so in launches of 36
+     * rows, 312 with 40 and one grid); then the fewest entries that still give
+     * that many slices, so that the last is not short (512 x 32,000: 95.7 -> 88.5) */
+    auto ept_for = [&](int g) {
+        const int e = (vocab + g * T - 1) / (g * T);
+        return e <= 16 ? 16 : e <= 24 ? 24 : e <= 32 ? 32 : e <= 40 || vocab <= 40 * T * kFullMaxG ? 40 : 48;
+    };
     int G = (512 + rows - 1) / rows;
     if (G > kFullMaxG) G = kFullMaxG;
-    if (G < 1) G = 1;
-    int ept = (vocab + G * T - 1) / (G * T);
-    ept = ept <= 16 ? 16 : ept <= 24 ? 24 : ept <= 32 ? 32 : ept <= 40 ? 40 : 48;
+    int ept = ept_for(G);
     G = (vocab + ept * T - 1) / (ept * T);
     if (G > kFullMaxG) return 1;
+    ept = ept_for(G);
     const int S = ept * T;
     if (p.n_out > S) return 1;
     /* (the no-wait test instance: 24 elements per thread, no soft-cap) */
@@ -338,20 +346,21 @@ int launch_full(dlk::RowParams &p, int rows, int vocab, int force_exact, int no_
         cap = dlk_full_kernel_capacity(ept, lds, softcap, hp);
         if (n_cap < 256) cap_cache[n_cap++] = CapEntry{dev, ept, lds, softcap, hp, cap};
     }
-    int rows_per = cap / G;
-    if (rows_per < 1) return 1;
-    if (rows_per > rows) rows_per = rows;
+    if (cap < G) return 1;                             /* a row's workgroups are not resident together */
     /* per row: the fallback's aggregates, then the row's values for the split
      * sums (V) or one slice's for a re-walked draw (S, which may exceed V) */
     const size_t fb_q_off = r16(aggs_bytes(vocab));
     const size_t fb_bytes = fb_q_off + r16((size_t)(vocab > S ? vocab : S) * 4);
+    /* rows per launch: as many as the workspace's bound holds */
+    const size_t room = g_noalloc ? kScratchBytes - kScratchCtrWords * 4 - 256 : kFullWorkspace;
+    const size_t per = fb_bytes + (size_t)G * kLaneWords * 8;
+    int rows_per = room / per < (size_t)rows ? (int)(room / per) : rows;
     if (g_noalloc) {
-        /* the fixed scratch array: as many rows per launch as it holds */
-        const size_t room = kScratchBytes - kScratchCtrWords * 4 - 256;
-        const size_t per = fb_bytes + (size_t)G * kLaneWords * 8;
-        if (room / per < (size_t)rows_per) rows_per = (int)(room / per);
-        if (rows_per < 1) return DLK_ERR_UNSUPPORTED;
+        const size_t words = kSyncWords + (size_t)G * kPubWords * 2;
+        if (kScratchCtrWords / words < (size_t)rows_per) rows_per = (int)(kScratchCtrWords / words);
     }
+    if (rows_per < rows && rows_per > 8) rows_per &= ~7;
+    if (rows_per < 1) return g_noalloc ? DLK_ERR_UNSUPPORTED : 1;
     const size_t n_ln = r16((size_t)rows_per * G * kLaneWords * 8);
     WsView ws;
     /* the published words live in the zeroed counter region: they are zero
@@ -368,6 +377,7 @@ int launch_full(dlk::RowParams &p, int rows, int vocab, int force_exact, int no_
     for (int r0 = 0; r0 < rows; r0 += rows_per) {
         const int nr = rows - r0 < rows_per ? rows - r0 : rows_per;
         f.p = rows_from(p, r0);
+        f.halves = nr % 8 == 0 && G % 2 == 0 && nr * G <= cap;
         if (dlk_launch_full_kernel(&f, nr, ept, lds, stream) != 0) return DLK_ERR_HIP;
     }
     return DLK_OK;

@@ -495,8 +495,9 @@ __global__ __launch_bounds__(kFullThreads) void full_kernel(FullParams f) {
     const RowParams &p = f.p;
     const int G = f.G, T = kFullThreads;
     /* a row's workgroups on one XCD: dispatch deals workgroup b to XCD b % 8,
-     * so when the grid holds whole groups of eight rows, the rows of b % 8 are
-     * those of XCD b % 8.  Among an XCD's blocks, the first half are the first
+     * so for whole groups of eight rows, the rows of b % 8 are those of XCD
+     * b % 8.  With halves (a grid that is resident at once, of whole groups of
+     * eight rows): among an XCD's blocks, the first half are the first
      * block of their CU and the second half the second (two per CU), and the
      * second block of a CU runs behind the first (older waves win issue): so a
      * row takes half its slices from each half, rather than all of a row's
@@ -504,7 +505,8 @@ __global__ __launch_bounds__(kFullThreads) void full_kernel(FullParams f) {
      * draw, the row's longest draw phase) and the last G/2 - 1 slices (where
      * the top-p crossing of a spread-out row lies, which the others wait for) */
     int row, g;
-    if (gridDim.x % (8 * G) == 0 && (G & 1) == 0) {
+    const int rows8 = ((int)gridDim.x / G) & ~7;   /* rows of whole groups of eight */
+    if (f.halves) {
         /* k: the block's place among its XCD's blocks; the first and second
          * halves of them are the first and second block of their CUs: each row
          * takes G/2 slices from each half */
@@ -513,7 +515,7 @@ __global__ __launch_bounds__(kFullThreads) void full_kernel(FullParams f) {
         row = (k2 / h) * 8 + (blockIdx.x & 7);
         const int i = k2 % h;
         g = k < R ? (i == 0 ? 0 : G - h + i) : 1 + i;
-    } else if (gridDim.x % (8 * G) == 0) {
+    } else if ((int)blockIdx.x < rows8 * G) {
         const int k = blockIdx.x >> 3;
         row = (k / G) * 8 + (blockIdx.x & 7);
         g = k % G;
@@ -1616,13 +1618,16 @@ extern "C" int dlk_launch_full_kernel(const dlk::FullParams *f, int rows, int ep
         if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) != hipSuccess) return -1;
         set[cap][hp - 1][which] = 1;
     }
-    /* An ordinary launch: the grid fits the device's resident workgroups
-     * (checked by the host against dlk_full_kernel_capacity), and the row
-     * waits only on workgroups of its own row.  Workgroups are dispatched in
-     * index order and a row's workgroups are consecutive, so every row below
-     * the dispatch frontier is fully resident and finishes, which frees room
-     * for the rest: the barriers make progress without a cooperative launch
-     * (which costs ~12 us of launch latency here), and every wait is bounded. */
+    /* An ordinary launch (a cooperative one costs ~12 us of launch latency
+     * here), of any number of rows: a workgroup waits only on workgroups of its
+     * own row.  With `halves` the host has checked that the whole grid is
+     * resident at once (dlk_full_kernel_capacity).  Otherwise the grid may be
+     * larger: each XCD is dealt its workgroups in index order, and on each XCD
+     * every workgroup of an earlier row (of the XCD's rows, or of all rows where
+     * they are spread) has the lower index, so the workgroups of the first row
+     * that is not finished are always the next to get a place, never behind
+     * those of a later row: it finishes, and by induction so do all.  Every wait
+     * is bounded besides. */
     FullParams fp = *f;
     void *args[] = {&fp};
     if (hipLaunchKernel(fn, dim3(rows * f->G), dim3(kFullThreads), args, lds, stream) != hipSuccess) return -1;

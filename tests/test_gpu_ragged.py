@@ -86,3 +86,14 @@ def test_topk_ragged(cuda, V, rows):
         if i == 3:
             w.softcap = 20.0
         run(w, 0, (i + 1) % 4)
+
+
+@pytest.mark.parametrize("rows,V", [(203, 65536), (516, 20480), (129, 40961), (96, 151936)])
+@pytest.mark.parametrize("path", [0, 2])
+def test_full_vocab_grids_past_the_resident_workgroups(cuda, rows, V, path):
+    """Grids of more workgroups than the device holds at once, of whole groups of eight rows and not, with and
+    without every row's exact fallbacks."""
+    rng = np.random.default_rng(rows)
+    lg = rng.normal(0, 2, size=(rows, V)).astype(np.float32)
+    hist = [rng.integers(0, V, 33) for _ in range(rows)]
+    run(make(f"grid-{rows}-{V}", rows, V, seed=rows, logits=lg, top_p=0.92, temperature=0.9, hist=hist, rep=1.2), path, 0)
