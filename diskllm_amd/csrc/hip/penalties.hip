@@ -22,6 +22,7 @@
 #include <mutex>
 
 #include "../../../include/diskllm_amd.h"
+#include "../host/dropin.h"
 
 namespace dlk {
 
@@ -112,6 +113,14 @@ __global__ __launch_bounds__(kPenThreads) void penalties_kernel(float *logits, i
     }
 }
 
+/* One op on compact values with their counts, a thread per distinct id (the
+ * drop-in penalty calls: vals and counts are pinned host memory, read and written
+ * over PCIe, so the call is one launch and no copies). */
+__global__ void compact_penalty_kernel(float *vals, const int32_t *counts, int n, uint32_t op, float value) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) vals[i] = penalize_ops(vals[i], counts[i], op, value, value, value);
+}
+
 /* After the sampling of a long-history call: the flagged rows get id -1, the
  * status bit and their rng state back (the sampling drew for them). */
 __global__ void long_history_fixup_kernel(int rows, const int32_t *too_long, const uint64_t *rng_saved,
@@ -170,6 +179,13 @@ extern "C" int dlk_launch_long_history_penalties(float *logits, int64_t ld, int 
                                                  const uint64_t *rng, uint64_t *rng_saved, hipStream_t stream) {
     return dlk::launch_penalties(logits, ld, rows, vocab, hist_off, hist_ids, order, rep, freq, pres,
                                  dlk::pen_slots(max_hist), max_hist, too_long, rng, rng_saved, stream);
+}
+
+extern "C" int dlk_launch_compact_penalty(float *vals, const int32_t *counts, int n, uint32_t op, float value,
+                                          hipStream_t stream) {
+    hipLaunchKernelGGL(dlk::compact_penalty_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, vals,
+                       counts, n, op, value);
+    return hipGetLastError() == hipSuccess ? DLK_OK : DLK_ERR_HIP;
 }
 
 extern "C" int dlk_launch_long_history_fixup(int rows, const int32_t *too_long, const uint64_t *rng_saved,

@@ -10,10 +10,10 @@
 int dlk_dropin_init(dlk_dropin_ctx *c) {
     memset(c, 0, sizeof(*c));
     if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess) return -1;
-    if (hipMalloc((void **)&c->hoff, 2 * sizeof(int32_t)) != hipSuccess) goto fail;
     if (hipMalloc((void **)&c->rng, sizeof(uint64_t)) != hipSuccess) goto fail;
     if (hipMalloc((void **)&c->ids, 2 * sizeof(int32_t)) != hipSuccess) goto fail;
     if (hipMalloc((void **)&c->status, sizeof(uint32_t)) != hipSuccess) goto fail;
+    if (hipHostMalloc((void **)&c->res, sizeof(*c->res), hipHostMallocDefault) != hipSuccess) goto fail;
     return 0;
 fail:
     dlk_dropin_release(c);
@@ -26,18 +26,19 @@ void dlk_dropin_release(dlk_dropin_ctx *c) {
         (void)dlk_release_stream(c->stream);
     }
     hipFree(c->logits);
-    hipFree(c->hist);
-    hipFree(c->hoff);
     hipFree(c->rng);
     hipFree(c->ids);
     hipFree(c->status);
     hipFree(c->mask);
+    if (c->res) hipHostFree(c->res);
+    if (c->pin) hipHostFree(c->pin);
     if (c->stream) hipStreamDestroy(c->stream);
     memset(c, 0, sizeof(*c));
 }
 
-int dlk_dropin_reserve(dlk_dropin_ctx *c, int vocab, int hist) {
+int dlk_dropin_reserve(dlk_dropin_ctx *c, int vocab) {
     if (vocab > c->cap) {
+        vocab = vocab > 0x7ffffff0 ? vocab : (vocab + 3) / 4 * 4;      /* staged in groups of four */
         hipStreamSynchronize(c->stream);
         hipFree(c->logits);
         hipFree(c->mask);
@@ -49,14 +50,21 @@ int dlk_dropin_reserve(dlk_dropin_ctx *c, int vocab, int hist) {
         c->cap = vocab;
         c->mask_cap = (vocab + 31) / 32;
     }
-    if (hist > c->hist_cap) {
-        hipStreamSynchronize(c->stream);
-        hipFree(c->hist);
-        c->hist = NULL;
-        c->hist_cap = 0;
-        if (hipMalloc((void **)&c->hist, (size_t)hist * sizeof(int32_t)) != hipSuccess) return -1;
-        c->hist_cap = hist;
+    return 0;
+}
+
+int dlk_dropin_reserve_pinned(dlk_dropin_ctx *c, size_t bytes) {
+    if (bytes <= c->pin_cap) return 0;
+    hipStreamSynchronize(c->stream);
+    if (c->pin) hipHostFree(c->pin);
+    c->pin = NULL;
+    c->pin_cap = 0;
+    bytes = (bytes + 4095) & ~(size_t)4095;
+    if (hipHostMalloc((void **)&c->pin, bytes, hipHostMallocDefault) != hipSuccess) {
+        c->pin = NULL;
+        return -1;
     }
+    c->pin_cap = bytes;
     return 0;
 }
 

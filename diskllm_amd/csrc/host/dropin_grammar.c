@@ -166,7 +166,7 @@ int diskllm_grammar_apply_mask(diskllm_grammar *g, float *logits, int vocab_size
         g->dev_ready = 1;
     }
     const int changed = read_table(g, vocab_size, tok_ctx, get_token_str);
-    if (changed < 0 || dlk_dropin_reserve(&g->dev, vocab_size, 0) != 0) return -1;
+    if (changed < 0 || dlk_dropin_reserve(&g->dev, vocab_size) != 0) return -1;
     hipStream_t st = g->dev.stream;
     if (changed) {
         hipStreamSynchronize(st);

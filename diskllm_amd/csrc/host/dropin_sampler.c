@@ -68,13 +68,21 @@ static int host_greedy(const float *logits, int vocab) {
  * greedy); -1 when a device call fails. */
 static int sample_one(dlk_dropin_ctx *c, const float *logits, int vocab, float temperature, int top_k, float top_p,
                       float min_p, int path, const uint64_t *rng, uint64_t *rng_out, uint32_t *status) {
-    if (dlk_dropin_reserve(c, vocab, 0) != 0) return -1;
+    const size_t row_bytes = (size_t)vocab * sizeof(float);
+    if (dlk_dropin_reserve(c, vocab) != 0 || dlk_dropin_reserve_pinned(c, row_bytes + 16) != 0) return -1;
     const int greedy = temperature == 0.0f;
-    if (hipMemcpyAsync(c->logits, logits, (size_t)vocab * sizeof(float), hipMemcpyHostToDevice, c->stream) !=
-        hipSuccess)
-        return -1;
-    if (!greedy &&
-        hipMemcpyAsync(c->rng, rng, sizeof(uint64_t), hipMemcpyHostToDevice, c->stream) != hipSuccess)
+    /* the row through pinned memory in two parts, so that the second is copied
+     * on the host while the device takes the first */
+    float *pin = (float *)c->pin;
+    const int half = vocab / 2 & ~3;
+    c->res->rng = *rng;
+    if (half > 0) {
+        memcpy(pin, logits, (size_t)half * sizeof(float));
+        if (dlk_launch_stage_row(c->logits, pin, half, NULL, NULL, NULL, c->stream) != DLK_OK) return -1;
+    }
+    memcpy(pin + half, logits + half, (size_t)(vocab - half) * sizeof(float));
+    if (dlk_launch_stage_row(c->logits + half, pin + half, vocab - half, c->res, c->rng, c->status, c->stream) !=
+        DLK_OK)
         return -1;
     dlk_batch b;
     memset(&b, 0, sizeof(b));
@@ -91,19 +99,12 @@ static int sample_one(dlk_dropin_ctx *c, const float *logits, int vocab, float t
     p.min_p = min_p;
     p.repeat_penalty = 1.0f;
     p.path = path;
-    if (hipMemsetAsync(c->status, 0, sizeof(uint32_t), c->stream) != hipSuccess) return -1;
     if (dlk_sample(&b, 1, vocab, &p, c->stream) != DLK_OK) return -1;
-    int32_t id = -1;
-    uint32_t st = 0;
-    if (hipMemcpyAsync(&id, c->ids, sizeof(int32_t), hipMemcpyDeviceToHost, c->stream) != hipSuccess) return -1;
-    if (hipMemcpyAsync(&st, c->status, sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream) != hipSuccess) return -1;
-    uint64_t r = 0;
-    if (!greedy && hipMemcpyAsync(&r, c->rng, sizeof(uint64_t), hipMemcpyDeviceToHost, c->stream) != hipSuccess)
-        return -1;
+    if (dlk_launch_publish_result(c->res, c->rng, c->ids, c->status, c->stream) != DLK_OK) return -1;
     if (hipStreamSynchronize(c->stream) != hipSuccess) return -1;
-    *status = st;
-    if (!greedy) *rng_out = r;
-    return id;
+    *status = c->res->status;
+    if (!greedy) *rng_out = c->res->rng;
+    return c->res->id;
 }
 
 /* The reference always returns a token (src/sampler.c:136-234): its caller
@@ -151,62 +152,48 @@ int greedy_sample(const float *logits, int vocab_size) {
     return id;
 }
 
-/* One penalty op in place on the host row.  Only the touched entries cross
- * PCIe: the logits of the distinct in-range ids (ids outside [0, vocab) are
- * skipped, as the reference skips them) go up as a compact row, the history as
- * slots of that row, the device applies the op there, and the compact row comes
- * back to be written over those ids: 12 bytes per id each way in place of the
- * whole row.  The order of a history does not matter to either op: repetition
- * scales an entry once per occurrence (its sign never changes), presence
- * subtracts once per distinct id. */
-typedef struct { int32_t id, pos; } id_pos;
-
-static int cmp_id_pos(const void *a, const void *b) {
-    const id_pos *x = (const id_pos *)a, *y = (const id_pos *)b;
-    if (x->id != y->id) return x->id < y->id ? -1 : 1;
-    return x->pos < y->pos ? -1 : x->pos > y->pos;
-}
-
+/* One penalty op in place on the host row.  Only the touched entries leave the
+ * host: the logits of the distinct in-range ids (ids outside [0, vocab) are
+ * skipped, as the reference skips them) and their counts go into pinned memory,
+ * a kernel applies the op to them there, and the values are written back over
+ * those ids: 12 bytes per id over PCIe in place of the whole row.  The order of a
+ * history does not matter to either op: repetition scales an entry once per
+ * occurrence (its sign never changes), presence subtracts once per distinct id. */
 static void report_penalty_failure(uint32_t op) {
     fprintf(stderr, "libdiskllm_amd: sampler_apply_%s_penalty could not reach the GPU; the row was not "
                     "penalised\n", op == DLK_OP_REPETITION ? "repetition" : "presence");
 }
 
 static void penalty_one(float *logits, int vocab, const int *seen, int n, uint32_t op, float value) {
-    id_pos *ip = malloc((size_t)n * sizeof(id_pos));
-    int32_t *slots = malloc((size_t)n * sizeof(int32_t));
+    size_t slots = 64;                              /* hash slots: at most half of them used */
+    while (slots < 2 * (size_t)n) slots <<= 1;
+    int32_t *table = calloc(slots, sizeof(int32_t));   /* entry d + 1 of the distinct ids, 0 = free */
     int32_t *ids = malloc((size_t)n * sizeof(int32_t));
-    float *vals = malloc((size_t)n * sizeof(float));
-    int m = 0, nd = 0;
-    if (ip && slots && ids && vals) {
-        for (int i = 0; i < n; i++)
-            if (seen[i] >= 0 && seen[i] < vocab) ip[m++] = (id_pos){seen[i], i};
-        qsort(ip, (size_t)m, sizeof(id_pos), cmp_id_pos);
-        for (int j = 0; j < m; j++) {
-            if (j == 0 || ip[j].id != ip[j - 1].id) {
-                ids[nd] = ip[j].id;
-                vals[nd] = logits[ip[j].id];
-                nd++;
-            }
-            slots[j] = nd - 1;
-        }
-    }
-    int done = nd == 0 && (ip && slots && ids && vals);
-    dlk_dropin_ctx *c = nd ? dlk_dropin_shared_lock() : NULL;
+    dlk_dropin_ctx *c = table && ids ? dlk_dropin_shared_lock() : NULL;
+    int done = 0;
     if (c) {
-        if (dlk_dropin_reserve(c, nd, m) == 0) {
-            const int32_t hoff[2] = {0, m};
-            const size_t bytes = (size_t)nd * sizeof(float);
-            int ok = hipMemcpyAsync(c->logits, vals, bytes, hipMemcpyHostToDevice, c->stream) == hipSuccess &&
-                     hipMemcpyAsync(c->hist, slots, (size_t)m * sizeof(int32_t), hipMemcpyHostToDevice,
-                                    c->stream) == hipSuccess &&
-                     hipMemcpyAsync(c->hoff, hoff, sizeof(hoff), hipMemcpyHostToDevice, c->stream) == hipSuccess;
-            if (ok)
-                ok = dlk_apply_penalties(c->logits, nd, 1, nd, c->hoff, c->hist, op,
-                                         op == DLK_OP_REPETITION ? value : 1.0f, 0.0f,
-                                         op == DLK_OP_PRESENCE ? value : 0.0f, c->stream) == DLK_OK;
-            if (ok) ok = hipMemcpyAsync(vals, c->logits, bytes, hipMemcpyDeviceToHost, c->stream) == hipSuccess;
-            if (hipStreamSynchronize(c->stream) == hipSuccess && ok) {
+        if (dlk_dropin_reserve_pinned(c, (size_t)n * (sizeof(float) + sizeof(int32_t))) == 0) {
+            float *vals = (float *)c->pin;
+            int32_t *counts = (int32_t *)c->pin + n;
+            int nd = 0;
+            for (int i = 0; i < n; i++) {
+                const int id = seen[i];
+                if (id < 0 || id >= vocab) continue;
+                size_t h = ((uint32_t)id * 0x9E3779B1u) & (slots - 1);
+                while (table[h] && ids[table[h] - 1] != id) h = (h + 1) & (slots - 1);
+                if (table[h]) {
+                    counts[table[h] - 1]++;
+                } else {
+                    ids[nd] = id;
+                    vals[nd] = logits[id];
+                    counts[nd] = 1;
+                    table[h] = ++nd;
+                }
+            }
+            const int ok = nd == 0 || dlk_launch_compact_penalty(vals, counts, nd, op, value, c->stream) == DLK_OK;
+            if (nd == 0) {
+                done = 1;
+            } else if (hipStreamSynchronize(c->stream) == hipSuccess && ok) {
                 for (int d = 0; d < nd; d++) logits[ids[d]] = vals[d];
                 done = 1;
             }
@@ -217,10 +204,8 @@ static void penalty_one(float *logits, int vocab, const int *seen, int n, uint32
      * only when host or device memory runs out or the GPU is gone: said on
      * stderr rather than passed over in silence */
     if (!done) report_penalty_failure(op);
-    free(ip);
-    free(slots);
+    free(table);
     free(ids);
-    free(vals);
 }
 
 void sampler_apply_repetition_penalty(float *logits, int vocab_size, const int *seen_tokens, int num_seen,
