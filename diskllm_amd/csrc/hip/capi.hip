@@ -15,6 +15,7 @@
 #include "sampler_params.h"
 #include "sampler_topk.h"
 #include "sampler_full.h"
+#include "tanhf_glibc.h"
 
 extern "C" int dlk_launch_row_kernel(const dlk::RowParams *p, int rows, size_t lds_bytes, hipStream_t stream);
 extern "C" int dlk_launch_topk_kernel(const dlk::TopkParams *f, int rows, size_t lds, hipStream_t stream);
@@ -316,6 +317,7 @@ int launch_full(dlk::RowParams &p, int rows, int vocab, int force_exact, int no_
     f.S = S;
     f.force_exact = force_exact;
     f.no_wait = no_wait;
+    f.cap_recip = dlk_softcap_recip(p.cap);
     /* carve order of full_kernel: sbits, ce, cbh, ca, rtot, rend, rpre, Pc, smap, svals, spx, elist, elc, seg,
      * tab, tbase, rres, rbase, pc, misc, md; 48 chunks staged per workgroup (sharp rows stage many: every
      * chunk with a tie and those around r's crossing) */

@@ -33,6 +33,8 @@ DLK_DEV float4 load4(const float *p) {
     return make_float4(x.x, x.y, x.z, x.w);
 }
 
+DLK_DEV void store4(float *p, float4 v) { *(f4_any *)p = f4_any{v.x, v.y, v.z, v.w}; }
+
 DLK_DEV uint64_t ballot(bool p) { return __ballot(p); }
 DLK_DEV int first_lane(uint64_t m) { return m ? __builtin_ctzll(m) : 64; }
 

@@ -50,6 +50,7 @@ struct FullParams {
     RowParams p;
     int G;             /* workgroups per row */
     int S;             /* slice length = EPT * kFullThreads */
+    float cap_recip;   /* dlk_softcap_recip(p.cap) */
     int halves;        /* block -> (row, slice): each row's slices from both halves of its XCD's blocks */
     int stage_cap;     /* chunks of final probabilities kept in LDS per workgroup */
     uint32_t *sync;    /* [rows][kSyncWords] */

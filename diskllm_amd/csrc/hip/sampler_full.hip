@@ -38,6 +38,7 @@
  */
 #include "sampler_common.h"
 #include "sampler_full.h"
+#include "softcap4.h"
 
 namespace dlk {
 
@@ -688,10 +689,7 @@ __global__ __launch_bounds__(kFullThreads) void full_kernel(FullParams f) {
     for (int j4 = 0; j4 < EPT / 4; j4++) {
         const int i0 = s0 + 4 * (t + j4 * T);
         float xs[4] = {raw[j4].x, raw[j4].y, raw[j4].z, raw[j4].w};
-        if (CAP) {
-#pragma unroll
-            for (int c = 0; c < 4; c++) xs[c] = dlk_softcap_glibc(xs[c], p.cap);
-        }
+        if (CAP) softcap4(xs, p.cap, f.cap_recip);
         if (i0 >= s1) xs[0] = xs[1] = xs[2] = xs[3] = -INFINITY;
         if (mk) {
             const uint32_t mw = mwd[j4] >> (i0 & 31);

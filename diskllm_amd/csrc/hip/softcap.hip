@@ -5,51 +5,44 @@
  * where it is a host loop over the vocabulary).  tanhf is bit-identical to the
  * host libm's (tanhf_glibc.h).
  *
- * HBM-bound elementwise work: 8 bytes per element (read + write).  Rows whose
- * stride and base allow it are processed as float4 (16-byte loads and stores);
- * a workgroup covers 4 * 256 * kSoftcapVec4 elements of one row.
+ * Elementwise work of 8 bytes per element (read + write) that the general form's
+ * 80 vector instructions per element made VALU-bound: 512 x 262,144 took 260-270 us
+ * where a copy of that size takes 208.  A group of four whose quotients lie in the
+ * common range in every lane takes the branch-free form instead: 207 us.  Rows
+ * of any alignment take 16-byte loads and stores (4-byte alignment is enough); a
+ * workgroup covers 4 * 256 * kSoftcapVec4 elements of one row.
  */
 #include <hip/hip_runtime.h>
 
-#include "tanhf_glibc.h"
+#include "softcap4.h"
 #include "../../../include/diskllm_amd.h"
 
 namespace dlk {
 
 constexpr int kSoftcapThreads = 256;
-constexpr int kSoftcapVec4 = 2;             /* float4 groups per thread */
+constexpr int kSoftcapVec4 = 1;             /* groups of four per thread (2: 216 us, 4: 221 at 512 x 262,144) */
 
 __global__ __launch_bounds__(kSoftcapThreads) void softcap_vec_kernel(float *__restrict__ logits, int64_t ld,
-                                                                      int vocab, float cap) {
+                                                                      int vocab, float cap, float recip) {
     float *row = logits + (int64_t)blockIdx.y * ld;
     const int base = (blockIdx.x * kSoftcapVec4 * kSoftcapThreads + threadIdx.x) * 4;
     float4 v[kSoftcapVec4];
 #pragma unroll
     for (int k = 0; k < kSoftcapVec4; k++) {
         const int i = base + k * kSoftcapThreads * 4;
-        if (i + 3 < vocab) v[k] = *(const float4 *)(row + i);
+        if (i + 3 < vocab) v[k] = load4(row + i);
     }
 #pragma unroll
     for (int k = 0; k < kSoftcapVec4; k++) {
         const int i = base + k * kSoftcapThreads * 4;
         if (i + 3 < vocab) {
-            float4 o;
-            o.x = dlk_softcap_glibc(v[k].x, cap);
-            o.y = dlk_softcap_glibc(v[k].y, cap);
-            o.z = dlk_softcap_glibc(v[k].z, cap);
-            o.w = dlk_softcap_glibc(v[k].w, cap);
-            *(float4 *)(row + i) = o;
+            float x[4] = {v[k].x, v[k].y, v[k].z, v[k].w};
+            softcap4(x, cap, recip);
+            store4(row + i, make_float4(x[0], x[1], x[2], x[3]));
         } else {
             for (int c = 0; c < 4 && i + c < vocab; c++) row[i + c] = dlk_softcap_glibc(row[i + c], cap);
         }
     }
-}
-
-__global__ __launch_bounds__(kSoftcapThreads) void softcap_scalar_kernel(float *__restrict__ logits, int64_t ld,
-                                                                         int vocab, float cap) {
-    float *row = logits + (int64_t)blockIdx.y * ld;
-    for (int i = blockIdx.x * kSoftcapThreads + threadIdx.x; i < vocab; i += gridDim.x * kSoftcapThreads)
-        row[i] = dlk_softcap_glibc(row[i], cap);
 }
 
 }  // namespace dlk
@@ -59,17 +52,9 @@ extern "C" int dlk_softcap(float *logits, int64_t ld, int rows, int vocab, float
     if (rows > 65535 || vocab > 0x7fffffff - 8192) return DLK_ERR_UNSUPPORTED;   /* grid rows; int indices */
     /* the reference caps only when the model's cap is positive (a NaN cap too is no cap) */
     if (rows == 0 || vocab == 0 || !(cap > 0.0f)) return DLK_OK;
-    const bool vec = ld % 4 == 0 && ((uintptr_t)logits & 15u) == 0;
-    if (vec) {
-        const int per = 4 * dlk::kSoftcapVec4 * dlk::kSoftcapThreads;
-        const dim3 grid((unsigned)((vocab + per - 1) / per), (unsigned)rows);
-        hipLaunchKernelGGL(dlk::softcap_vec_kernel, grid, dim3(dlk::kSoftcapThreads), 0, stream, logits, ld, vocab,
-                           cap);
-    } else {
-        int bx = (vocab + dlk::kSoftcapThreads - 1) / dlk::kSoftcapThreads;
-        if (bx > 1024) bx = 1024;
-        hipLaunchKernelGGL(dlk::softcap_scalar_kernel, dim3((unsigned)bx, (unsigned)rows),
-                           dim3(dlk::kSoftcapThreads), 0, stream, logits, ld, vocab, cap);
-    }
+    const int per = 4 * dlk::kSoftcapVec4 * dlk::kSoftcapThreads;
+    const dim3 grid((unsigned)((vocab + per - 1) / per), (unsigned)rows);
+    hipLaunchKernelGGL(dlk::softcap_vec_kernel, grid, dim3(dlk::kSoftcapThreads), 0, stream, logits, ld, vocab, cap,
+                       dlk_softcap_recip(cap));
     return hipGetLastError() == hipSuccess ? DLK_OK : DLK_ERR_HIP;
 }

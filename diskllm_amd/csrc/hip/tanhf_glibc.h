@@ -126,4 +126,75 @@ DLK_TH float dlk_tanhf_glibc(float x) {
 /* The reference's soft-cap of one logit: cap * tanhf(x / cap). */
 DLK_TH float dlk_softcap_glibc(float x, float cap) { return cap * dlk_tanhf_glibc(x / cap); }
 
+/* ---- the same for the common range, branch-free --------------------------------
+ * For q = |x / cap| in [2^-60, 0.75 ln2) tanhf takes -t / (t + 2) with
+ * t = expm1f(-2 q), and that takes k = 0 (2 q <= ln2 / 2) or k = -1: two forms
+ * that differ by a constant and a final scaling, so both are computed without a
+ * branch (with k = 0 the correction c is 0 and x * (e - c) - c is x * e; below
+ * 2^-25, where expm1f returns its argument, x + x^2 / 2 rounds to x).  Every
+ * operation keeps its value and its order; what is left out is the divisions'
+ * scaling for operands near the ends of the exponent range, which do not occur:
+ * the 80 vector instructions of the general form are about 60. */
+
+/* n / d correctly rounded, for normal n, d and quotient well inside the exponent
+ * range: the division sequence of the hardware without its scaling and fix-up
+ * (reciprocal, one Newton step, quotient, two remainder corrections). */
+DLK_TH float dlk_div_inner(float n, float d) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    const float y0 = __builtin_amdgcn_rcpf(d);
+#else
+    const float y0 = 1.0f / d;
+#endif
+    const float y = __builtin_fmaf(__builtin_fmaf(-d, y0, 1.0f), y0, y0);
+    const float q0 = n * y;
+    const float q1 = __builtin_fmaf(__builtin_fmaf(-d, q0, n), y, q0);
+    return __builtin_fmaf(__builtin_fmaf(-d, q1, n), y, q1);
+}
+
+/* What the caps need of cap: its reciprocal rounded to float, with which two
+ * remainder corrections round x / cap correctly (Markstein's theorem: a
+ * correctly rounded reciprocal of a divisor whose significand is not all ones),
+ * or 0 where that is not given and the general form is taken. */
+DLK_TH float dlk_softcap_recip(float cap) {
+    const uint32_t u = dlk_th_f2u(cap);
+    if (!(cap >= 0x1p-20f && cap <= 0x1p40f) || (u & 0x7fffffu) == 0x7fffffu) return 0.0f;
+    return (float)(1.0 / (double)cap);
+}
+
+/* |x / cap| (recip from dlk_softcap_recip; meaningful where dlk_softcap_common holds) */
+DLK_TH float dlk_softcap_quot(float x, float cap, float recip) {
+    const float a = __builtin_fabsf(x);
+    const float q0 = a * recip;
+    const float q1 = __builtin_fmaf(__builtin_fmaf(-cap, q0, a), recip, q0);
+    return __builtin_fmaf(__builtin_fmaf(-cap, q1, a), recip, q1);
+}
+
+/* q's place above the lower end of the common range; the form below holds where
+ * this is under DLK_SOFTCAP_SPAN (unsigned: NaN, 0 and everything outside is not). */
+#define DLK_SOFTCAP_SPAN (0x3f051592u - 0x21800000u)
+DLK_TH uint32_t dlk_softcap_place(float q) { return dlk_th_f2u(q) - 0x21800000u; }
+
+/* cap * tanhf(x / cap) for q = |x / cap| in the common range. */
+DLK_TH float dlk_softcap_common(float x, float q, float cap) {
+    const float kLn2Hi = dlk_th_u2f(0x3f317180u), kLn2Lo = dlk_th_u2f(0x3717f7d1u);
+    const float kQ1 = dlk_th_u2f(0xbd088889u), kQ2 = dlk_th_u2f(0x3ad00d01u), kQ3 = dlk_th_u2f(0xb8a670cdu),
+                kQ4 = dlk_th_u2f(0x36867e54u), kQ5 = dlk_th_u2f(0xb457edbbu);
+    const float x2 = -2.0f * q;
+    const int low = -x2 > dlk_th_u2f(0x3eb17218u);     /* k = -1 */
+    const float hi = x2 + (low ? kLn2Hi : 0.0f);
+    const float lo = low ? -kLn2Lo : 0.0f;
+    const float r = hi - lo;
+    const float c = (hi - r) - lo;
+    const float hfx = 0.5f * r;
+    const float hxs = r * hfx;
+    const float r1 = 1.0f + hxs * (kQ1 + hxs * (kQ2 + hxs * (kQ3 + hxs * (kQ4 + hxs * kQ5))));
+    const float t = 3.0f - r1 * hfx;
+    float e = hxs * dlk_div_inner(r1 - t, 6.0f - r * t);
+    e = r * (e - c) - c;
+    e -= hxs;
+    const float y0 = r - e;
+    const float y = low ? 0.5f * y0 - 0.5f : y0;
+    return __builtin_copysignf(cap * dlk_div_inner(-y, y + 2.0f), x);
+}
+
 #endif
