@@ -174,7 +174,7 @@ bool workspace(hipStream_t stream, int kind, size_t counters, size_t data_bytes,
 }
 
 size_t fixed_lds(const dlk::LdsPlan &pl) {
-    return r16(32 * 8) + r16(64 * 8) + r16(16 * 8) + r16(64 * 4) + 4 * r16((size_t)pl.hcap * 4) +
+    return r16(32 * 8) + r16(64 * 8) + r16(16 * 8) + r16(64 * 4) + 4 * r16((size_t)pl.hfix * 4) +
            r16((size_t)pl.flag_words * 4);
 }
 
@@ -281,14 +281,15 @@ int launch_topk(dlk::RowParams &p, int rows, int vocab, hipStream_t stream) {
 
 /* Fused full-vocabulary path (sampler_full.hip): DLK_OK, or 1 when outside its
  * range (the caller then uses the row kernel). */
-int launch_full(dlk::RowParams &p, int rows, int vocab, int force_exact, int no_wait, hipStream_t stream) {
+int launch_full(dlk::RowParams p, int rows, int vocab, int max_hist, int force_exact, int no_wait,
+                hipStream_t stream) {
     using namespace dlk;
     const int T = kFullThreads;
     if (p.greedy || p.topk_on || p.s_general) return 1;
     /* min-p with the cut after the first kept entry (it may lie in any slice): the row kernel */
     if (p.minp_on && p.topp_on && p.top_p <= 0.0f) return 1;
     if (!(p.inv_temp < INFINITY)) return 1;            /* (v - M) * inv_t is NaN at the maximum */
-    if (p.plan.hcap > 2 * T) return 1;                 /* one or two history ids per thread, loaded first */
+    if (p.plan.hcap > kFullHistPer * T) return 1;      /* the history's ids in registers, loaded first */
     if (((uintptr_t)p.logits & 3) != 0) return 1;      /* (rows of any stride and length: load4) */
     if (vocab < 8192) return 1;                        /* not one workgroup's slice */
     /* about 512 workgroups, two per CU on 256 CUs, and no more than 40 entries
@@ -311,12 +312,17 @@ int launch_full(dlk::RowParams &p, int rows, int vocab, int force_exact, int no_
     /* (the no-wait test instance: 24 elements per thread, no soft-cap) */
     if (no_wait && (ept != 24 || p.cap > 0.0f)) return DLK_ERR_UNSUPPORTED;
     const int nch = S / 64;
+    /* past 512 ids the history's arrays share the LDS of the draw's staged chunks
+     * where they fit, so that two workgroups still fit a CU (64 x 151,936 with
+     * 1,000 ids: 88 -> 54 us) */
+    p.plan.hfix = p.plan.hcap > kFullThreads && p.plan.hcap <= kHcapDirect ? 0 : p.plan.hcap;
     FullParams f;
     memset(&f, 0, sizeof(f));
     f.G = G;
     f.S = S;
     f.force_exact = force_exact;
     f.no_wait = no_wait;
+    f.max_hist = max_hist;
     f.cap_recip = dlk_softcap_recip(p.cap);
     /* carve order of full_kernel: sbits, ce, cbh, ca, rtot, rend, rpre, Pc, smap, svals, spx, elist, elc, seg,
      * tab, tbase, rres, rbase, pc, misc, md; 48 chunks staged per workgroup (sharp rows stage many: every
@@ -349,6 +355,11 @@ int launch_full(dlk::RowParams &p, int rows, int vocab, int force_exact, int no_
         if (n_cap < 256) cap_cache[n_cap++] = CapEntry{dev, ept, lds, softcap, hp, cap};
     }
     if (cap < G) return 1;                             /* a row's workgroups are not resident together */
+    /* past kHcapDirect ids the table's LDS leaves one workgroup per CU, which
+     * costs a larger grid as much as the pre-pass does (two rounds of 44 us
+     * against 44 + 40 at 64 rows of 151,936); a grid resident at once takes such
+     * histories here (16 rows of 128,256 and 3,000 ids: 49 -> 32 us) */
+    if (p.plan.hcap > kHcapDirect && (int64_t)rows * G > cap) return 1;
     /* per row: the fallback's aggregates, then the row's values for the split
      * sums (V) or one slice's for a re-walked draw (S, which may exceed V) */
     const size_t fb_q_off = r16(aggs_bytes(vocab));
@@ -422,7 +433,41 @@ int sample_impl(const dlk_batch *b, int rows, int vocab, const dlk_sample_params
     if (!greedy && !b->rng) return DLK_ERR_INVALID;
     const int max_hist = prm->max_history > 0 ? prm->max_history : 1024;
     const bool cap_on = prm->softcap > 0.0f;                    /* src/core/context.c:604 */
-    if (b->hist_off && pow2_at_least(max_hist, 64) > kHcapDirect) {
+    dlk::RowParams p;
+    memset(&p, 0, sizeof(p));
+    p.logits = b->logits; p.ld = b->ld; p.V = vocab;
+    p.hist_off = b->hist_off; p.hist_ids = b->hist_ids;
+    p.mask = b->mask; p.mask_ld = b->mask_ld; p.mask_row = b->mask_row;
+    p.rng = b->rng; p.out_ids = b->out_ids;
+    p.out_cand_ids = b->out_cand_ids; p.out_cand_probs = b->out_cand_probs; p.out_cand_logprobs = b->out_cand_logprobs;
+    p.n_out = prm->n_out; p.status = b->status;
+    p.top_p = prm->top_p; p.min_p = prm->min_p;
+    p.rep = prm->repeat_penalty; p.freq = prm->frequency_penalty; p.pres = prm->presence_penalty;
+    p.order = prm->penalty_order;
+    p.greedy = greedy;
+    p.cap = cap_on ? prm->softcap : 0.0f;          /* applied inside the sampling kernels */
+    if (!p.greedy) {
+        p.inv_temp = 1.0f / prm->temperature;                   /* src/sampler.c:154 */
+        /* 1/T negative, zero or infinite: s = (l - max) * (1/T) may be NaN or +inf
+         * and its maximum is not 0; the row kernel handles it */
+        p.s_general = !(p.inv_temp > 0.0f && p.inv_temp < INFINITY);
+    }
+    p.topk_on = prm->top_k > 0 && prm->top_k < vocab;           /* src/sampler.c:166 */
+    p.top_k = prm->top_k;
+    p.topp_on = prm->top_p < 1.0f;                              /* src/sampler.c:205 */
+    p.topp_thr = (p.topp_on && prm->top_p > 0.0f) ? topp_threshold(prm->top_p) : 0.0;
+    p.minp_on = prm->min_p > 0.0f;                              /* src/sampler.c:188 */
+
+    dlk::LdsPlan &pl = p.plan;
+    pl.hcap = pl.hfix = b->hist_off ? pow2_at_least(max_hist, 64) : 64;
+    int nch = (vocab + 63) / 64;
+    pl.flag_words = (nch + 31) / 32;
+    if (b->hist_off && pl.hcap > kHcapDirect) {
+        /* the fused full-vocabulary kernel takes such histories itself where it can */
+        if ((prm->path == DLK_PATH_AUTO || prm->path == DLK_PATH_FULL_EXACT) && !p.greedy && !p.topk_on && !g_noalloc) {
+            const int rc = launch_full(p, rows, vocab, max_hist, prm->path == DLK_PATH_FULL_EXACT, 0, stream);
+            if (rc <= 0) return rc;
+        }
         /* a history too long to stage in LDS: the rows as sampler_sample would
          * see them -- soft-cap, mask, penalties (src/core/sampler_api.c:51-61) --
          * in a scratch copy; then the sampling alone over the copy.  A row whose
@@ -460,36 +505,6 @@ int sample_impl(const dlk_batch *b, int rows, int vocab, const dlk_sample_params
         return dlk_launch_long_history_fixup(rows, too_long, rng_saved, greedy ? nullptr : b->rng, b->out_ids,
                                              b->status, stream);
     }
-
-    dlk::RowParams p;
-    memset(&p, 0, sizeof(p));
-    p.logits = b->logits; p.ld = b->ld; p.V = vocab;
-    p.hist_off = b->hist_off; p.hist_ids = b->hist_ids;
-    p.mask = b->mask; p.mask_ld = b->mask_ld; p.mask_row = b->mask_row;
-    p.rng = b->rng; p.out_ids = b->out_ids;
-    p.out_cand_ids = b->out_cand_ids; p.out_cand_probs = b->out_cand_probs; p.out_cand_logprobs = b->out_cand_logprobs;
-    p.n_out = prm->n_out; p.status = b->status;
-    p.top_p = prm->top_p; p.min_p = prm->min_p;
-    p.rep = prm->repeat_penalty; p.freq = prm->frequency_penalty; p.pres = prm->presence_penalty;
-    p.order = prm->penalty_order;
-    p.greedy = greedy;
-    p.cap = cap_on ? prm->softcap : 0.0f;          /* applied inside the sampling kernels */
-    if (!p.greedy) {
-        p.inv_temp = 1.0f / prm->temperature;                   /* src/sampler.c:154 */
-        /* 1/T negative, zero or infinite: s = (l - max) * (1/T) may be NaN or +inf
-         * and its maximum is not 0; the row kernel handles it */
-        p.s_general = !(p.inv_temp > 0.0f && p.inv_temp < INFINITY);
-    }
-    p.topk_on = prm->top_k > 0 && prm->top_k < vocab;           /* src/sampler.c:166 */
-    p.top_k = prm->top_k;
-    p.topp_on = prm->top_p < 1.0f;                              /* src/sampler.c:205 */
-    p.topp_thr = (p.topp_on && prm->top_p > 0.0f) ? topp_threshold(prm->top_p) : 0.0;
-    p.minp_on = prm->min_p > 0.0f;                              /* src/sampler.c:188 */
-
-    dlk::LdsPlan &pl = p.plan;
-    pl.hcap = b->hist_off ? pow2_at_least(max_hist, 64) : 64;
-    int nch = (vocab + 63) / 64;
-    pl.flag_words = (nch + 31) / 32;
     const bool big_k = p.topk_on && !p.greedy && p.top_k > kMaxTopKLds;
     pl.kp = p.topk_on && !big_k ? pow2_at_least(p.top_k, 64) : 0;
     if (big_k) return launch_row_global_topk(p, rows, stream);
@@ -507,8 +522,8 @@ int sample_impl(const dlk_batch *b, int rows, int vocab, const dlk_sample_params
     }
     if ((prm->path == DLK_PATH_AUTO || prm->path == DLK_PATH_FULL_EXACT || prm->path == DLK_PATH_FULL_NO_WAIT) &&
         !p.greedy && !p.topk_on) {
-        int rc = launch_full(p, rows, vocab, prm->path == DLK_PATH_FULL_EXACT, prm->path == DLK_PATH_FULL_NO_WAIT,
-                             stream);
+        int rc = launch_full(p, rows, vocab, pl.hcap, prm->path == DLK_PATH_FULL_EXACT,
+                             prm->path == DLK_PATH_FULL_NO_WAIT, stream);
         if (rc <= 0) return rc;
     }
     if (total > kMaxLds) return DLK_ERR_UNSUPPORTED;

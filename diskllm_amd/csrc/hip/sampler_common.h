@@ -92,10 +92,10 @@ DLK_DEV Lds make_lds(unsigned char *base, const LdsPlan &pl) {
     L.red = (double *)carve(p, 64 * 8);
     L.bd = (double *)carve(p, 16 * 8);
     L.bi = (int *)carve(p, 64 * 4);
-    L.hsort = (uint32_t *)carve(p, (size_t)pl.hcap * 4);
-    L.pid = (int *)carve(p, (size_t)pl.hcap * 4);
-    L.pval = (float *)carve(p, (size_t)pl.hcap * 4);
-    L.pcnt = (int *)carve(p, (size_t)pl.hcap * 4);
+    L.hsort = (uint32_t *)carve(p, (size_t)pl.hfix * 4);
+    L.pid = (int *)carve(p, (size_t)pl.hfix * 4);
+    L.pval = (float *)carve(p, (size_t)pl.hfix * 4);
+    L.pcnt = (int *)carve(p, (size_t)pl.hfix * 4);
     L.pflag = (uint32_t *)carve(p, (size_t)pl.flag_words * 4);
     L.region = p;
     return L;

@@ -9,6 +9,7 @@
 namespace dlk {
 
 constexpr int kFullThreads = 512;    /* two workgroups per CU */
+constexpr int kFullHistPer = 8;      /* history ids per thread of the long-history instances */
 constexpr int kFullMaxG = 16;        /* workgroups per row */
 constexpr int kPubWords = 16;        /* 64-bit words each workgroup publishes */
 constexpr int kCandSlots = 2;        /* predicted top-p crossing chunks per workgroup */
@@ -50,6 +51,7 @@ struct FullParams {
     RowParams p;
     int G;             /* workgroups per row */
     int S;             /* slice length = EPT * kFullThreads */
+    int max_hist;      /* longer histories are flagged (DLK_STATUS_HISTORY_TOO_LONG) */
     float cap_recip;   /* dlk_softcap_recip(p.cap) */
     int halves;        /* block -> (row, slice): each row's slices from both halves of its XCD's blocks */
     int stage_cap;     /* chunks of final probabilities kept in LDS per workgroup */

@@ -487,8 +487,9 @@ __device__ __forceinline__ void draw_fix(const FullParams &f, int row, int h, ui
 
 /* NOWAIT (a test instance): every wait gives up at its first poll that finds a
  * word not yet written, which sets DLK_STATUS_SYNC_TIMEOUT. */
-/* HP: history ids per thread (1 up to kFullThreads ids; 2 up to twice that,
- * an instance of its own so that the common case keeps its registers). */
+/* HP: history ids per thread: 1 up to kFullThreads ids, kFullHistPer up to that
+ * many times as many (an instance of its own so that the common case keeps its
+ * registers and gathers its logits before the bulk loads). */
 template <int EPT, bool CAP, bool NOWAIT = false, int HP = 1>
 __global__ __launch_bounds__(kFullThreads) void full_kernel(FullParams f) {
     constexpr uint32_t kLimit = NOWAIT ? 0u : kFullSpinLimit;
@@ -558,6 +559,17 @@ __global__ __launch_bounds__(kFullThreads) void full_kernel(FullParams f) {
     int *misc = (int *)carve(q, 64 * 4);
     double *md = (double *)carve(q, 16 * 8);
     if (t < 32) L.tab[t] = kExp2Tab[t];
+    /* the history's arrays in the staged chunks' LDS (free until the top-p
+     * crossing, and again when a re-walked draw needs them) */
+    if (HP > 1 && p.plan.hfix == 0) {
+        const int hc = p.plan.hcap;
+        L.hsort = (uint32_t *)svals;
+        L.pid = (int *)(L.hsort + hc);
+        L.pval = (float *)(L.pid + hc);
+        L.pcnt = (int *)(L.pval + hc);
+    }
+    /* HP > 1: the table's slots owned by any entry (in the candidate tables' LDS) */
+    int *olist = (int *)tab;
 
     /* ---- history first: the row's ids (HP per thread; the host keeps the
      *      direct history within the workgroup) and, for an id inside this
@@ -569,17 +581,13 @@ __global__ __launch_bounds__(kFullThreads) void full_kernel(FullParams f) {
         nh = p.hist_off[row + 1] - p.hist_off[row];
     }
     int hid[HP];
-    float gx[HP];
-    uint32_t gm[HP];
+    float gx = 0.0f;
+    uint32_t gm = 0xffffffffu;
 #pragma unroll
-    for (int k = 0; k < HP; k++) {
-        hid[k] = t + k * T < nh ? hist[t + k * T] : -1;
-        gx[k] = 0.0f;
-        gm[k] = 0xffffffffu;
-        if (hid[k] >= s0 && hid[k] < s1) {
-            gx[k] = lg[hid[k]];
-            if (mk) gm[k] = mk[hid[k] >> 5];
-        }
+    for (int k = 0; k < HP; k++) hid[k] = t + k * T < nh ? hist[t + k * T] : -1;
+    if (HP == 1 && hid[0] >= s0 && hid[0] < s1) {
+        gx = lg[hid[0]];
+        if (mk) gm = mk[hid[0] >> 5];
     }
 
     /* ---- stream the slice into registers: every load issued before any use */
@@ -587,7 +595,7 @@ __global__ __launch_bounds__(kFullThreads) void full_kernel(FullParams f) {
     uint32_t mwd[EPT / 4];
     load_slice<EPT, 0, EPT / 4>(lg, mk, s0, s1, t, T, raw, mwd);
 
-    if (DLK_COLD(nh > p.plan.hcap || nh > HP * T)) {    /* (the host keeps both) */
+    if (DLK_COLD(nh > f.max_hist || nh > HP * T)) {    /* (the host keeps both) */
         if (g == 0 && t == 0) {
             p.out_ids[row] = -1;
             if (p.status) atomicOr(p.status, DLK_STATUS_HISTORY_TOO_LONG);
@@ -614,18 +622,21 @@ __global__ __launch_bounds__(kFullThreads) void full_kernel(FullParams f) {
     const int hshift = 32 - (31 - __clz(hslots));
     for (int i = t; i < nw; i += T) sbits[i] = 0;
     for (int i = t; i < hslots; i += T) { hkey[i] = -1; hcnt[i] = 0u; }
-    if (t == 0) { misc[5] = 0; misc[6] = 0; }     /* a NaN / +inf entry; a wait that gave up */
+    if (t == 0) { misc[4] = 0; misc[5] = 0; misc[6] = 0; }   /* owned slots; a NaN / +inf entry; a wait that gave up */
     __syncthreads();
-    int oslot[HP];
+    int oslot = -1;
 #pragma unroll
     for (int k = 0; k < HP; k++) {
-        oslot[k] = -1;
         const int id = hid[k];
         if (id >= s0 && id < s1) {
             uint32_t h = ((uint32_t)id * 0x9E3779B1u) >> hshift;
             for (int probe = 0; probe < hslots; probe++) {
                 const int old = atomicCAS(&hkey[h], -1, id);
-                if (old == -1) { oslot[k] = (int)h; atomicOr(&sbits[(id - s0) >> 5], 1u << ((id - s0) & 31)); }
+                if (old == -1) {
+                    if (HP == 1) oslot = (int)h;
+                    else olist[atomicAdd(&misc[4], 1)] = (int)h;
+                    atomicOr(&sbits[(id - s0) >> 5], 1u << ((id - s0) & 31));
+                }
                 if (old == -1 || old == id) break;
                 h = (h + 1) & (uint32_t)(hslots - 1);
             }
@@ -650,13 +661,21 @@ __global__ __launch_bounds__(kFullThreads) void full_kernel(FullParams f) {
         }
     }
     __syncthreads();
-#pragma unroll
-    for (int k = 0; k < HP; k++) {
-        if (oslot[k] >= 0) {
-            float x = gx[k];
+    if (HP == 1) {
+        if (oslot >= 0) {
+            float x = gx;
             if (CAP) x = dlk_softcap_glibc(x, p.cap);
-            if (!((gm[k] >> (hid[k] & 31)) & 1u)) x = -INFINITY;
-            hcnt[oslot[k]] = __float_as_uint(penalize(x, (int)hcnt[oslot[k]], p));
+            if (!((gm >> (hid[0] & 31)) & 1u)) x = -INFINITY;
+            hcnt[oslot] = __float_as_uint(penalize(x, (int)hcnt[oslot], p));
+        }
+    } else {
+        /* (a slice of a long history owns few of its ids: about one a thread) */
+        for (int i = t; i < misc[4]; i += T) {
+            const int h = olist[i], id = hkey[h];
+            float x = lg[id];
+            if (CAP) x = dlk_softcap_glibc(x, p.cap);
+            if (mk && !((mk[id >> 5] >> (id & 31)) & 1u)) x = -INFINITY;
+            hcnt[h] = __float_as_uint(penalize(x, (int)hcnt[h], p));
         }
     }
     if (DLK_COLD(tslot >= 0)) {
@@ -1590,8 +1609,9 @@ const void *full_fn_hp(int which) {
 }
 /* the instance for (elements per thread, soft-cap, history ids per thread) */
 const void *full_fn(int which, int cap, int hp) {
-    if (cap) return hp > 1 ? full_fn_hp<true, 2>(which) : full_fn_hp<true, 1>(which);
-    return hp > 1 ? full_fn_hp<false, 2>(which) : full_fn_hp<false, 1>(which);
+    constexpr int kH = dlk::kFullHistPer;
+    if (cap) return hp > 1 ? full_fn_hp<true, kH>(which) : full_fn_hp<true, 1>(which);
+    return hp > 1 ? full_fn_hp<false, kH>(which) : full_fn_hp<false, 1>(which);
 }
 int ept_index(int ept) { return ept == 16 ? 0 : ept == 24 ? 1 : ept == 32 ? 2 : ept == 40 ? 3 : ept == 48 ? 4 : -1; }
 }  // namespace

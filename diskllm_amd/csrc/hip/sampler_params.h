@@ -14,6 +14,7 @@ namespace dlk {
 /* LDS layout of the one-workgroup-per-row kernel. */
 struct LdsPlan {
     int hcap;        /* history sort capacity (power of two >= 64) */
+    int hfix;        /* entries of it in the kernel's fixed LDS: hcap, or 0 where the kernel places them */
     int flag_words;  /* words of the per-64-element "has a penalised id" bitmap */
     int kp;          /* top-k candidate capacity (power of two >= k), 0 if top-k is off */
     int bytes;       /* total dynamic LDS */
