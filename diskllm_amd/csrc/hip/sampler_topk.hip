@@ -61,7 +61,7 @@ DLK_DEV float penalised(const RowParams &p, float x, int cnt) {
  * slice is streamed and thresholded on its raw logits -- with +-inf clamped to
  * +-FLT_MAX, which the cap maps to the same +-cap -- and only the candidates it
  * collects are capped; the penalty patches are capped values, handled from
- * their LDS list.  Ties that the cap creates are resolved by the order
+ * their LDS table.  Ties that the cap creates are resolved by the order
  * (y desc, index asc) of the collected candidates and the merge's certificate. */
 
 /* A bound just below the r-th largest of the 128 ascending keys a, b held two per
@@ -100,29 +100,66 @@ DLK_DEV float4 load_group(const float *lg, int i0, int s1) {
     return x;
 }
 
+/* The slice's penalised ids: an LDS hash table (open addressing, at most half
+ * full) whose slots hold an id's count, then its penalised value.  Looked up, and
+ * walked slot by slot where every patch is wanted: a list of them searched from
+ * end to end per flagged group made the exact pass of a slice with some 200
+ * patches 80 us. */
+struct PatchTab {
+    int *key;                                      /* -1: free */
+    int *val;
+    int slots, shift;                              /* a power of two; 32 - log2(slots) */
+    DLK_DEV int find(int id) const {
+        uint32_t h = ((uint32_t)id * 0x9E3779B1u) >> shift;
+        while (true) {
+            const int k = key[h];
+            if (k == id) return (int)h;
+            if (k == -1) return -1;
+            h = (h + 1) & (uint32_t)(slots - 1);
+        }
+    }
+    DLK_DEV float value(int slot) const { return __int_as_float(val[slot]); }
+};
+
 /* Bits of the group at i0 whose entries come from the stream: inside the slice,
- * allowed by the mask word bits `mw` (already shifted to i0), not penalised.  A
- * penalised id sets its group's bit in gbits; such groups look their ids up in
- * the slice's patch list (pid[0 .. np)). */
-DLK_DEV uint32_t group_live(uint32_t mw, const uint32_t *gbits, const int *pid, int np, int i0, int s0, int s1) {
+ * allowed by the mask word bits `mw` (already shifted to i0), not penalised (a
+ * penalised id sets its group's bit in gbits).  AT_ONCE: for the greedy stream,
+ * where the lookups are on the slice's path (64 x 128,256: 16.4 -> 15.6 us); the
+ * other kinds look few groups up after it, and the longer code costs them 0.4 us. */
+template <bool AT_ONCE>
+DLK_DEV uint32_t group_live(uint32_t mw, const uint32_t *gbits, const PatchTab &pt, int i0, int s0, int s1) {
     uint32_t live = mw;
     if (i0 + 4 > s1) live &= i0 < s1 ? (1u << (s1 - i0)) - 1u : 0u;
     const int gr = (i0 - s0) >> 2;
-    if ((gbits[gr >> 5] >> (gr & 31)) & 1u)
-        for (int k = 0; k < np; k++) {
-            const unsigned d = (unsigned)(pid[k] - i0);
-            if (d < 4u) live &= ~(1u << d);
+    if ((gbits[gr >> 5] >> (gr & 31)) & 1u) {
+        if (AT_ONCE) {
+            /* the four first probes at once; most end there */
+            int k[4];
+            uint32_t more = 0;
+#pragma unroll
+            for (int c = 0; c < 4; c++) k[c] = pt.key[((uint32_t)(i0 + c) * 0x9E3779B1u) >> pt.shift];
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                if (k[c] == i0 + c) live &= ~(1u << c);
+                else if (k[c] != -1) more |= 1u << c;
+            }
+            for (more &= live; more; more &= more - 1) {
+                const int c = __builtin_ctz(more);
+                if (pt.find(i0 + c) >= 0) live &= ~(1u << c);
+            }
+        } else {
+#pragma unroll 1
+            for (int c = 0; c < 4; c++)
+                if (pt.find(i0 + c) >= 0) live &= ~(1u << c);
         }
+    }
     return live & 0xFu;
 }
 
 /* Whether id (inside the slice) is one of the penalised ids. */
-DLK_DEV bool is_patched(const uint32_t *gbits, const int *pid, int np, int id, int s0) {
+DLK_DEV bool is_patched(const uint32_t *gbits, const PatchTab &pt, int id, int s0) {
     const int gr = (id - s0) >> 2;
-    if (!((gbits[gr >> 5] >> (gr & 31)) & 1u)) return false;
-    for (int k = 0; k < np; k++)
-        if (pid[k] == id) return true;
-    return false;
+    return ((gbits[gr >> 5] >> (gr & 31)) & 1u) && pt.find(id) >= 0;
 }
 
 /* Bits of the group at i0 allowed by the mask word bits `mw` and inside the slice. */
@@ -175,8 +212,8 @@ DLK_DEV int keep_best(uint64_t *buf, int n, int r, int *slot) {
 /* The slice of a row that one workgroup streams: groups of four elements at
  * s0 + 4 * (t + j * T), j = 0 .. S/(4T) - 1, in batches of four groups per thread
  * with the next batch's loads in flight.
- *   - The penalised ids of the slice are patched from an LDS list (their stream
- *     entries count as -inf and the list is folded in afterwards).
+ *   - The penalised ids of the slice are patched from an LDS table (their stream
+ *     entries count as -inf and the patches are folded in afterwards).
  *   - Threshold: after batch 0 each wave takes the ceil(KP/4)-th largest of its
  *     lanes' two best group maxima (distinct entries, so the wave holds at least
  *     that many entries at or above it); the smallest of the four is a valid
@@ -274,83 +311,60 @@ __global__ __launch_bounds__(kTopkThreads, 8) void topk_kernel(TopkParams f) {
     }
     for (int i = t; i < f.S / 128; i += T) gbits[i] = 0;
     if (t < 16) misc[t] = 0;                       /* (16.. are written before they are read) */
-    int *hkey = (int *)L.hsort;                    /* the history's hash table (below), cleared while batch 0 lands */
-    int *hcnt = (int *)L.pval;
+    /* the penalised ids of the slice: its history entries are counted in the
+     * table (2 * hcap >= 2 * nh slots, so every id has its slot and probes stay
+     * short); the entry that inserted an id computes its patch once every count
+     * is in, in place of the count: the patch depends only on the id, its count,
+     * its logit and its mask word, so any one occurrence may compute it.  Their
+     * groups' bits go to gbits, misc[11] of them are allowed by the mask.  Keys
+     * span hsort and pid, values pval and pcnt (carved back to back, each hcap
+     * words, a multiple of 16 bytes).  Cleared here, while batch 0 lands. */
     const int hslots = 2 * p.plan.hcap;            /* a power of two */
+    const PatchTab pt{(int *)L.hsort, (int *)L.pval, hslots, 32 - (31 - __clz(hslots))};
     if (nh > 0)
-        for (int i = t; i < hslots; i += T) { hkey[i] = -1; hcnt[i] = 0; }
-
-    /* penalty patches of the ids inside this slice: misc[0] entries of
-     * (pid, pval), their groups' bits in gbits, misc[11] of them allowed by the
-     * mask.  The slice's history entries are counted in an LDS hash table of
-     * their ids (open addressing over 2 * hcap >= 2 * nh slots, so every id has
-     * its slot and probes stay short); the entry that inserted an id computes
-     * its patch once every count is in: the patch depends only on the id, its
-     * count, its logit and its mask word, so any one occurrence may compute it.
-     * Keys span hsort and pid, counts pval and pcnt (carved back to back, each
-     * hcap words, a multiple of 16 bytes); pid and pval are reused for the
-     * patch list only after the counts have been read. */
-    const int hshift = 32 - (31 - __clz(hslots));
-    constexpr int kPer = kTopkHcapMax / kTopkThreads;   /* history entries per thread (nh <= hcap) */
+        for (int i = t; i < hslots; i += T) { pt.key[i] = -1; pt.val[i] = 0; }
+    int *olist = (int *)cbuf;                      /* owned slots of the ids past the first T (hcap <= 2 * cand_cap) */
     auto count_patches = [&]() {
-        int oslot[kPer], oid[kPer];
-        float ov[kPer];
-        uint32_t om[kPer];
-        /* the first T entries from registers (read early), the rest loaded here */
-#pragma unroll
-        for (int k = 0; k < kPer; k++) {
-            const int i = t + k * T;
-            oslot[k] = -1;
-            oid[k] = -1;
-            ov[k] = 0.0f;
-            om[k] = 0xffffffffu;
-            if (i >= nh) continue;
-            const int id = k == 0 ? hid : hist[i];
-            if (id < s0 || id >= s1) continue;
-            oid[k] = id;
-            if (k == 0) {
-                ov[k] = hval;
-                om[k] = hmw;
-            } else {
-                ov[k] = lg[id];
-                om[k] = mk ? mk[id >> 5] : 0xffffffffu;
-            }
-            uint32_t h = ((uint32_t)id * 0x9E3779B1u) >> hshift;
-            bool found = false;
-            for (int probe = 0; probe < hslots && !found; probe++) {
-                const int old = atomicCAS(&hkey[h], -1, id);
-                if (old == -1) oslot[k] = (int)h;
-                if (old == -1 || old == id) found = true;
-                else h = (h + 1) & (uint32_t)(hslots - 1);
-            }
-            if (found) atomicAdd(&hcnt[h], 1);
-        }
-        __syncthreads();
-        int cnt[kPer];
-#pragma unroll
-        for (int k = 0; k < kPer; k++) cnt[k] = oslot[k] >= 0 ? hcnt[oslot[k]] : 0;
-        __syncthreads();                           /* counts read: pid and pval are free */
-#pragma unroll
-        for (int k = 0; k < kPer; k++) {
-            if (oslot[k] < 0) continue;
-            const int id = oid[k];
-            float v = ov[k];
-            const bool allowed = (om[k] >> (id & 31)) & 1u;
+        auto patch = [&](int h, int id, float v, uint32_t mw) {
+            const bool allowed = (mw >> (id & 31)) & 1u;
             if (CAP) v = dlk_softcap_glibc(v, p.cap);  /* the soft-cap first (src/core/context.c:873-876) */
             if (!allowed) v = -INFINITY;
-            v = penalised(p, v, cnt[k]);
-            const int at = atomicAdd(&misc[0], 1);
-            if (at < p.plan.hcap) { L.pid[at] = id; L.pval[at] = v; }
+            pt.val[h] = __float_as_int(penalised(p, v, pt.val[h]));
             if (allowed) atomicAdd(&misc[11], 1);
             atomicOr(&gbits[(id - s0) >> 7], 1u << (((id - s0) >> 2) & 31));
+        };
+        int oslot = -1;
+#pragma unroll 1
+        for (int i = t; i < nh; i += T) {
+            const int id = i == t ? hid : hist[i];
+            if (id < s0 || id >= s1) continue;
+            uint32_t h = ((uint32_t)id * 0x9E3779B1u) >> pt.shift;
+            int old = 0;
+            for (int probe = 0; probe < hslots; probe++) {
+                old = atomicCAS(&pt.key[h], -1, id);
+                if (old == -1 || old == id) break;
+                h = (h + 1) & (uint32_t)(hslots - 1);
+            }
+            if (old == -1) {
+                if (i == t) oslot = (int)h;
+                else olist[atomicAdd(&misc[0], 1)] = (int)h;
+            }
+            atomicAdd(&pt.val[h], 1);
         }
         __syncthreads();
+        if (oslot >= 0) patch(oslot, hid, hval, hmw);
+        if (nh > T)
+            for (int i = t; i < misc[0]; i += T) {
+                const int h = olist[i], id = pt.key[h];
+                patch(h, id, lg[id], mk ? mk[id >> 5] : 0xffffffffu);
+            }
+        __syncthreads();
     };
+    const int npt = nh > 0 ? hslots : 0;           /* slots to walk for every patch */
     if (GREEDY) {                                  /* greedy streams exact values */
         __syncthreads();
         if (nh > 0) count_patches();
     }
-    int np = GREEDY ? min(misc[0], p.plan.hcap) : 0;
 
     /* ---- 2. stream the slice -------------------------------------------- */
     float m1 = -INFINITY, m2 = -INFINITY;          /* the lane's two best group maxima */
@@ -367,7 +381,7 @@ __global__ __launch_bounds__(kTopkThreads, 8) void topk_kernel(TopkParams f) {
             /* (non-greedy: the penalised ids stream their raw logits; the
              * patches come after the stream) */
             const uint32_t mw = m[j] >> msh;
-            const uint32_t live = GREEDY ? group_live(mw, gbits, L.pid, np, i0, s0, s1) : range_live(mw, i0, s1);
+            const uint32_t live = GREEDY ? group_live<true>(mw, gbits, pt, i0, s0, s1) : range_live(mw, i0, s1);
             const float4 v = x[j];
             float e[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
@@ -443,9 +457,9 @@ __global__ __launch_bounds__(kTopkThreads, 8) void topk_kernel(TopkParams f) {
          *      lane's best group read again cost the last blocks 6 us) ------- */
         if (gi >= 0) bi = gi;
         bm = m1;
-        for (int k2 = t; k2 < np; k2 += T) {
-            const float y = L.pval[k2];
-            const int id = L.pid[k2];
+        for (int k2 = t; k2 < npt; k2 += T) {
+            const int id = pt.key[k2];
+            const float y = id >= 0 ? pt.value(k2) : -INFINITY;
             /* (a row whose maximum is -inf samples index 0: no index is taken then) */
             if (y > bm || (y == bm && y > -INFINITY && id < bi)) { bm = y; bi = id; }
         }
@@ -454,8 +468,10 @@ __global__ __launch_bounds__(kTopkThreads, 8) void topk_kernel(TopkParams f) {
             /* the reference compares from logits[0] (src/sampler.c:10-17): NaN there wins */
             float x0 = lg[0];
             if (mk && !(mk[0] & 1u)) x0 = -INFINITY;
-            for (int k2 = 0; k2 < np; k2++)
-                if (L.pid[k2] == 0) x0 = L.pval[k2];
+            if (npt) {
+                const int at = pt.find(0);
+                if (at >= 0) x0 = pt.value(at);
+            }
             fnan = isnan(x0) ? 1u : 0u;
         }
     } else {
@@ -473,11 +489,11 @@ __global__ __launch_bounds__(kTopkThreads, 8) void topk_kernel(TopkParams f) {
         }
         /* (the table was cleared before the stream's first barrier) */
         if (nh > 0) count_patches();
-        np = nh > 0 ? min(misc[0], p.plan.hcap) : 0;
         float pmax = -INFINITY;
         int pn = 0, pirr = 0;
-        for (int k2 = t; k2 < np; k2 += T) {       /* the patches: capped values under CAP */
-            const float y = L.pval[k2];
+        for (int k2 = t; k2 < npt; k2 += T) {      /* the patches: capped values under CAP */
+            if (pt.key[k2] < 0) continue;
+            const float y = pt.value(k2);
             pn += y > -INFINITY;
             pirr |= !(y < INFINITY) && !(y == -INFINITY);
             pmax = fmaxf(pmax, y);
@@ -507,7 +523,7 @@ __global__ __launch_bounds__(kTopkThreads, 8) void topk_kernel(TopkParams f) {
                 const int i0 = s0 + 4 * k2;
                 const float4 v = load_group(lg, i0, s1);
                 const uint32_t live =
-                    group_live(mk && i0 < s1 ? mk[i0 >> 5] >> (i0 & 31) : 0xFu, gbits, L.pid, np, i0, s0, s1);
+                    group_live<GREEDY>(mk && i0 < s1 ? mk[i0 >> 5] >> (i0 & 31) : 0xFu, gbits, pt, i0, s0, s1);
                 const float e[4] = {v.x, v.y, v.z, v.w};
                 float gmx = -INFINITY;
                 for (int c = 0; c < 4; c++) {
@@ -558,7 +574,7 @@ __global__ __launch_bounds__(kTopkThreads, 8) void topk_kernel(TopkParams f) {
                 const int i0 = all_groups ? s0 + 4 * k2 : (int)grp[k2];
                 if (i0 >= s1) continue;
                 const float4 v = load_group(lg, i0, s1);
-                const uint32_t live = group_live(mk ? mk[i0 >> 5] >> (i0 & 31) : 0xFu, gbits, L.pid, np, i0, s0, s1);
+                const uint32_t live = group_live<GREEDY>(mk ? mk[i0 >> 5] >> (i0 & 31) : 0xFu, gbits, pt, i0, s0, s1);
                 const float e[4] = {v.x, v.y, v.z, v.w};
                 for (int c = 0; c < 4; c++) {
                     float y = e[c];
@@ -569,11 +585,13 @@ __global__ __launch_bounds__(kTopkThreads, 8) void topk_kernel(TopkParams f) {
                     }
                 }
             }
-            for (int k2 = t; k2 < np; k2 += T) {
-                const float y = L.pval[k2];
+            for (int k2 = t; k2 < npt; k2 += T) {
+                const int id = pt.key[k2];
+                if (id < 0) continue;
+                const float y = pt.value(k2);
                 if (y > -INFINITY && y >= cte) {
                     const int at = atomicAdd(&misc[10], 1);
-                    if (at < f.cand_cap) cbuf[at] = ((uint64_t)desc_key(y) << 32) | (uint32_t)L.pid[k2];
+                    if (at < f.cand_cap) cbuf[at] = ((uint64_t)desc_key(y) << 32) | (uint32_t)id;
                 }
             }
             __syncthreads();
@@ -603,7 +621,7 @@ __global__ __launch_bounds__(kTopkThreads, 8) void topk_kernel(TopkParams f) {
                 for (int i = t; i < C; i += T) {
                     const uint64_t e = cbuf[i];
                     const uint32_t id = (uint32_t)e;
-                    if (!is_patched(gbits, L.pid, np, (int)id, s0)) {
+                    if (!is_patched(gbits, pt, (int)id, s0)) {
                         const float y = dlk_softcap_glibc(key_value((uint32_t)(e >> 32)), p.cap);
                         cbuf[i] = ((uint64_t)desc_key(y) << 32) | id;
                     }

@@ -54,3 +54,29 @@ def test_greedy_first_of_equal_maxima(cuda, rows, V):
         lg[r, at] = np.float32(20)
         hist.append([int(at.min())] if r % 3 == 0 else [int(rng.integers(0, V))])
     run_and_check(make(f"greedy-{rows}", rows, V, seed=rows, logits=lg, temperature=0.0, rep=1.5, hist=hist), 0)
+
+
+@pytest.mark.parametrize("n", [255, 257, 642, 1024])
+@pytest.mark.parametrize("kw", [dict(top_k=31, temperature=0.8, top_p=0.9), dict(temperature=0.0), dict(top_k=9)])
+def test_topk_many_patches(cuda, n, kw):
+    """Hundreds of penalised ids in a slice, among them its best entries (the exact pass over its groups), ids that
+    share a group or a hash chain, and ids repeated through the history."""
+    rows, V = 24, 48896
+    rng = np.random.default_rng(n)
+    lg = rng.normal(0, 2.5, size=(rows, V)).astype(np.float32)
+    hist = []
+    for r in range(rows):
+        kind = r % 4
+        h = rng.integers(0, V, n)
+        if kind == 1:
+            h = np.argsort(-lg[r])[:n]                 # the row's best entries
+        elif kind == 2:
+            h = 4096 + np.arange(n)                    # neighbours, whole groups
+        elif kind == 3:
+            h = rng.integers(0, 50, n) * 256           # repeats
+        hist.append(h)
+    w = make(f"patches-{n}", rows, V, seed=n, logits=lg, hist=hist, rep=1.29, pres=0.2, **kw)
+    run_and_check(w, 0)
+    if kw.get("top_k") == 9:
+        w.softcap = 30.0
+        run_and_check(w, 0)
