@@ -68,8 +68,6 @@ __device__ __forceinline__ void load_slice(const float *lg, const uint32_t *mk, 
 }
 
 
-constexpr int kClassNanPosInf = 1 | 2 | 512;       /* signalling NaN, quiet NaN, +inf */
-
 DLK_DEV float wave_max(float v) { return wave_max_dpp(v); }
 
 /* Published words carry kReady (bit 63; every value stored in them leaves it
@@ -622,7 +620,7 @@ __global__ __launch_bounds__(kFullThreads) void full_kernel(FullParams f) {
     const int hshift = 32 - (31 - __clz(hslots));
     for (int i = t; i < nw; i += T) sbits[i] = 0;
     for (int i = t; i < hslots; i += T) { hkey[i] = -1; hcnt[i] = 0u; }
-    if (t == 0) { misc[4] = 0; misc[5] = 0; misc[6] = 0; }   /* owned slots; a NaN / +inf entry; a wait that gave up */
+    if (t == 0) { misc[4] = 0; misc[5] = 0; misc[6] = 0; }   /* owned slots; a NaN entry; a wait that gave up */
     __syncthreads();
     int oslot = -1;
 #pragma unroll
@@ -703,13 +701,14 @@ __global__ __launch_bounds__(kFullThreads) void full_kernel(FullParams f) {
      * the row's last group, where it is not whole) */
     float v[EPT];
     float tm = -INFINITY;
-    bool bad = false;                              /* NaN or +inf after penalties */
+    const bool whole = s0 + S <= V;                /* (uniform) */
+    bool bad = false;                              /* NaN after penalties (+inf shows in the maximum) */
 #pragma unroll
     for (int j4 = 0; j4 < EPT / 4; j4++) {
         const int i0 = s0 + 4 * (t + j4 * T);
         float xs[4] = {raw[j4].x, raw[j4].y, raw[j4].z, raw[j4].w};
         if (CAP) softcap4(xs, p.cap, f.cap_recip);
-        if (i0 >= s1) xs[0] = xs[1] = xs[2] = xs[3] = -INFINITY;
+        if (!whole && i0 >= s1) xs[0] = xs[1] = xs[2] = xs[3] = -INFINITY;
         if (mk) {
             const uint32_t mw = mwd[j4] >> (i0 & 31);
 #pragma unroll
@@ -717,7 +716,7 @@ __global__ __launch_bounds__(kFullThreads) void full_kernel(FullParams f) {
                 if (!((mw >> c) & 1u)) xs[c] = -INFINITY;
         }
         const int li0 = i0 - s0;
-        const uint32_t pb = i0 < s1 ? (sbits[li0 >> 5] >> (li0 & 31)) & 0xFu : 0u;
+        const uint32_t pb = (sbits[li0 >> 5] >> (li0 & 31)) & 0xFu;
         if (pb) {
             /* the patched ids of the group (src/sampler.c:21-52) */
 #pragma unroll
@@ -728,8 +727,8 @@ __global__ __launch_bounds__(kFullThreads) void full_kernel(FullParams f) {
         for (int c = 0; c < 4; c++) {
             v[j4 * 4 + c] = xs[c];
             tm = fmaxf(tm, xs[c]);
-            bad |= __builtin_amdgcn_class(xs[c], kClassNanPosInf);
         }
+        bad |= __builtin_isunordered(xs[0], xs[1]) | __builtin_isunordered(xs[2], xs[3]);
     }
     if (ballot(bad) != 0 && lane == 0) misc[5] = 1;
 
@@ -753,7 +752,7 @@ __global__ __launch_bounds__(kFullThreads) void full_kernel(FullParams f) {
     }
     if (g == 0 && t == 0) p.rng[row] = st;                  /* every workgroup has read it */
     const int n_out = p.n_out;
-    if (DLK_COLD(row_bad || !(M > -INFINITY))) {
+    if (DLK_COLD(row_bad || !(M > -INFINITY && M < INFINITY))) {
         /* every entry -inf, or a NaN / +inf entry: the softmax sum is NaN, no
          * comparison with it holds, and the draw falls through to index V-1 */
         if (g == 0) {
@@ -796,8 +795,10 @@ __global__ __launch_bounds__(kFullThreads) void full_kernel(FullParams f) {
     /* |sequential - exact| <= V u sum; |ours - exact| <= 64 u sum (summation depth) */
     const double U = 0x1p-53;
     const double eps_s = ((double)V + 64.0) * U * 1.01 + 4.0 * U;
-    const float inv_a = (float)(1.0 / (Sapx * (1.0 + eps_s)));
-    const float inv_b = (float)(1.0 / (Sapx * (1.0 - eps_s)));
+    /* 1 / (S (1 +- eps)) lies within 1 / S (1 -+ e2): one division */
+    const double rS = 1.0 / Sapx, e2 = eps_s * (1.0 + 0x1p-20) + 0x1p-51;
+    const float inv_a = (float)(rS * (1.0 - e2));
+    const float inv_b = (float)(rS * (1.0 + e2));
     bool ok = inv_a == inv_b && !f.force_exact;
     float inv = inv_a;
     if (DLK_COLD((inv_a != inv_b || f.force_exact) && !misc[6])) {
@@ -947,7 +948,9 @@ __global__ __launch_bounds__(kFullThreads) void full_kernel(FullParams f) {
             const int idx[2] = {kPubP, kPubP0};
             row_gather<kLimit>(pubrow, G, idx, pc, p.status, &misc[6]);
         }
-        for (int h = 0; h < g; h++) RWg += u2d(pc[h * kPubWords + kPubP]);
+        /* the slices' prefixes, one per lane (every wave, G <= 64) */
+        const double Rl = wave_incl_scan_d(lane < G ? u2d(pc[lane * kPubWords + kPubP]) : 0.0);
+        if (g > 0) RWg = u2d(readlane64(d2u(Rl), g - 1));
         const double U = 0x1p-53;
         int hx = -1;                               /* the slice that finds x */
         if (!topp) {
@@ -959,24 +962,19 @@ __global__ __launch_bounds__(kFullThreads) void full_kernel(FullParams f) {
             /* the first slice whose end prefix may reach tau; |ours - sequential|
              * within the bound e of the reference's double sum (src/sampler.c:209) */
             const double tau = p.topp_thr;
-            double R = 0.0;
-            bool amb = false;
-            for (int h = 0; h < G && hx < 0; h++) {
-                R += u2d(pc[h * kPubWords + kPubP]);
-                const double e = ((double)min(V, (h + 1) * S) + 256.0) * U * 1.01 + 4.0 * U;
-                if (R * (1.0 + e) >= tau) {
-                    hx = h;
-                    amb = R * (1.0 - e) < tau;     /* the crossing may be at its very end or beyond */
-                }
-            }
-            if (hx < 0) {
+            const double e = ((double)min(V, (lane + 1) * S) + 256.0) * U * 1.01 + 4.0 * U;
+            const uint64_t reach = ballot(lane < G && Rl * (1.0 + e) >= tau);
+            const uint64_t below = ballot(Rl * (1.0 - e) < tau);
+            if (reach) {
+                hx = __builtin_ctzll(reach);
+                if ((below >> hx) & 1) ok = false; /* the crossing may be at its very end or beyond */
+            } else {
                 /* the whole row stays below top_p: nk = k (src/sampler.c:208-215) */
-                const double e = ((double)V + 256.0) * U * 1.01 + 4.0 * U;
-                const float a = (float)(1.0 / (R * (1.0 + e))), b = (float)(1.0 / (R * (1.0 - e)));
+                const double R = u2d(readlane64(d2u(Rl), G - 1));
+                const double eV = ((double)V + 256.0) * U * 1.01 + 4.0 * U;
+                const float a = (float)(1.0 / (R * (1.0 + eV))), b = (float)(1.0 / (R * (1.0 - eV)));
                 if (a == b) inv3 = a;
                 else ok = false;
-            } else if (amb) {
-                ok = false;
             }
         }
         if (ok && hx == g) {
@@ -1002,26 +1000,29 @@ __global__ __launch_bounds__(kFullThreads) void full_kernel(FullParams f) {
             if (c1 >= 0 && c1 < c0) { const int tmp = c0; c0 = c1; c1 = tmp; }
             /* each candidate's exact prefix: the slice's values before it, summed
              * per thread and over the block; and its 64 values into LDS */
-            double m0 = 0.0, m1 = 0.0;
             float *cv = svals;
+            auto prefix_to = [&](int cc, int at) {
+                double m = 0.0;
 #pragma unroll
-            for (int j4 = 0; j4 < EPT / 4; j4++) {
-                const int u = t + j4 * T;           /* 4-element group index */
-                const double d = ((double)v[4 * j4] + (double)v[4 * j4 + 1]) + ((double)v[4 * j4 + 2] + (double)v[4 * j4 + 3]);
-                if (u < 16 * c0) m0 += d;
-                if (u < 16 * c1) m1 += d;
-                const int cg = u >> 4;
-                if (okc && (cg == c0 || cg == c1))
-                    *(float4 *)&cv[(cg == c0 ? 0 : 64) + (u & 15) * 4] =
-                        make_float4(v[4 * j4], v[4 * j4 + 1], v[4 * j4 + 2], v[4 * j4 + 3]);
-            }
-            m0 = wave_incl_scan_d(m0);
-            m1 = wave_incl_scan_d(m1);
-            if (lane == 63) { L.red[wave_id()] = m0; L.red[32 + wave_id()] = m1; }
+                for (int j4 = 0; j4 < EPT / 4; j4++) {
+                    const int u = t + j4 * T;       /* 4-element group index */
+                    const double d = ((double)v[4 * j4] + (double)v[4 * j4 + 1]) + ((double)v[4 * j4 + 2] + (double)v[4 * j4 + 3]);
+                    if (u < 16 * cc) m += d;
+                    if (okc && (u >> 4) == cc)
+                        *(float4 *)&cv[at + (u & 15) * 4] =
+                            make_float4(v[4 * j4], v[4 * j4 + 1], v[4 * j4 + 2], v[4 * j4 + 3]);
+                }
+                m = wave_incl_scan_d(m);
+                if (lane == 63) L.red[at / 2 + wave_id()] = m;
+            };
+            prefix_to(c0, 0);
+            if (DLK_COLD(c1 >= 0)) prefix_to(c1, 64);
             __syncthreads();
             if (wave_id() == 0) {
                 double P0 = 0.0, P1 = 0.0;
-                for (int w2 = 0; w2 < T / 64; w2++) { P0 += L.red[w2]; P1 += L.red[32 + w2]; }
+                for (int w2 = 0; w2 < T / 64; w2++) P0 += L.red[w2];
+                if (c1 >= 0)
+                    for (int w2 = 0; w2 < T / 64; w2++) P1 += L.red[32 + w2];
                 int xx = V - 1;
                 double s3 = 0.0, eps3 = 0.0;
                 bool found = false;
@@ -1043,8 +1044,9 @@ __global__ __launch_bounds__(kFullThreads) void full_kernel(FullParams f) {
                 float i3 = 1.0f;
                 if (!found) okc = 0;
                 if (okc) {
-                    const float a = (float)(1.0 / (s3 * (1.0 + eps3)));
-                    const float b = (float)(1.0 / (s3 * (1.0 - eps3)));
+                    const double r3 = 1.0 / s3, e3 = eps3 * (1.0 + 0x1p-20) + 0x1p-51;
+                    const float a = (float)(r3 * (1.0 - e3));
+                    const float b = (float)(r3 * (1.0 + e3));
                     if (a == b) i3 = a;
                     else okc = 0;
                 }
