@@ -718,10 +718,16 @@ __global__ __launch_bounds__(kFullThreads) void full_kernel(FullParams f) {
         const int li0 = i0 - s0;
         const uint32_t pb = (sbits[li0 >> 5] >> (li0 & 31)) & 0xFu;
         if (pb) {
-            /* the patched ids of the group (src/sampler.c:21-52) */
-#pragma unroll
-            for (int c = 0; c < 4; c++)
-                if ((pb >> c) & 1u) xs[c] = hpatch(i0 + c);
+            /* the patched ids of the group (src/sampler.c:21-52), one at a time:
+             * a lookup per entry made this loop's code three times as long */
+            for (uint32_t rest = pb; rest; rest &= rest - 1) {
+                const int c = __builtin_ctz(rest);
+                const float y = hpatch(i0 + c);
+                xs[0] = c == 0 ? y : xs[0];
+                xs[1] = c == 1 ? y : xs[1];
+                xs[2] = c == 2 ? y : xs[2];
+                xs[3] = c == 3 ? y : xs[3];
+            }
         }
 #pragma unroll
         for (int c = 0; c < 4; c++) {
@@ -1136,7 +1142,7 @@ __global__ __launch_bounds__(kFullThreads) void full_kernel(FullParams f) {
 #pragma unroll
     for (int j = 0; j < EPT; j++) {
         const int i = s0 + 4 * (t + (j / 4) * T) + (j & 3);
-        v[j] = i <= x ? (topp ? v[j] * inv3 : v[j]) : 0.0f;
+        v[j] = i <= x ? v[j] * inv3 : 0.0f;        /* (inv3 is 1 without top-p) */
     }
     /* (a uniform test first: the log must not be evaluated speculatively when
      * no log-probabilities are asked for) */
