@@ -156,6 +156,10 @@ bool workspace(hipStream_t stream, int kind, size_t counters, size_t data_bytes,
         cc = (cc + 63) & ~(size_t)63;
         size_t db = w->data_bytes > data_bytes ? w->data_bytes : data_bytes;
         if (db < (1u << 20)) db = 1u << 20;
+        /* no allocation while the stream is captured: it would end the capture */
+        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(stream, &cs) != hipSuccess) (void)hipGetLastError();
+        else if (cs != hipStreamCaptureStatusNone) return false;
         if (w->ptr) {
             /* the stream's earlier kernels may still use the old buffer */
             if (hipStreamSynchronize(stream) != hipSuccess) return false;
@@ -194,6 +198,11 @@ dlk::RowParams rows_from(const dlk::RowParams &p, int r0) {
     if (p.out_cand_logprobs) q.out_cand_logprobs = p.out_cand_logprobs + (int64_t)r0 * p.n_out;
     return q;
 }
+
+/* Rows that are not whole 16-byte groups: where no workspace can be had for the
+ * fused kernels (the fixed array is too small, or the stream is being captured
+ * and holds none yet) they run on the row kernel, which needs none. */
+bool row_kernel_instead(const dlk::RowParams &p) { return ((uintptr_t)p.logits & 15) != 0 || (p.ld & 3) != 0; }
 
 /* Single-pass top-k path (sampler_topk.hip): returns DLK_OK, or 1 when the
  * configuration is outside its range (the caller then uses the row kernel). */
@@ -272,7 +281,7 @@ int launch_topk(dlk::RowParams &p, int rows, int vocab, hipStream_t stream) {
     size_t n_slot = r16((size_t)rows * G * sizeof(TopkSlot));
     size_t n_cand = (size_t)rows * G * KP * 8;
     WsView ws;
-    if (!workspace(stream, 0, (size_t)rows, n_slot + n_cand, ws)) return g_ws_err;
+    if (!workspace(stream, 0, (size_t)rows, n_slot + n_cand, ws)) return row_kernel_instead(p) ? 1 : g_ws_err;
     f.counters = ws.counters;
     f.slots = (TopkSlot *)ws.data;
     f.cands = (uint64_t *)(ws.data + n_slot);
@@ -373,14 +382,14 @@ int launch_full(dlk::RowParams p, int rows, int vocab, int max_hist, int force_e
         if (kScratchCtrWords / words < (size_t)rows_per) rows_per = (int)(kScratchCtrWords / words);
     }
     if (rows_per < rows && rows_per > 8) rows_per &= ~7;
-    if (rows_per < 1) return g_noalloc ? DLK_ERR_UNSUPPORTED : 1;
+    if (rows_per < 1) return g_noalloc && !row_kernel_instead(p) && (vocab & 3) == 0 ? DLK_ERR_UNSUPPORTED : 1;
     const size_t n_ln = r16((size_t)rows_per * G * kLaneWords * 8);
     WsView ws;
     /* the published words live in the zeroed counter region: they are zero
      * between launches (the kernel returns them to zero) */
     if (!workspace(stream, 0, (size_t)rows_per * kSyncWords + (size_t)rows_per * G * kPubWords * 2,
                    n_ln + (size_t)rows_per * fb_bytes, ws))
-        return g_ws_err;
+        return row_kernel_instead(p) || (vocab & 3) != 0 ? 1 : g_ws_err;
     f.sync = ws.counters;
     f.pub = (uint64_t *)(ws.counters + (size_t)rows_per * kSyncWords);
     f.lanes = (uint64_t *)ws.data;

@@ -60,7 +60,7 @@ typedef struct {
     float presence_penalty;   /* active when != 0 */
     uint32_t penalty_order;   /* DLK_ORDER_* or any packing of DLK_OP_* */
     int max_history;          /* upper bound on any row's history length (0 = 1024); above 1024 the
-                                 penalties are applied to a scratch copy of the rows first */
+                                 penalties may be applied to a scratch copy of the rows first */
     int n_out;                /* candidate outputs per row (0 = none) */
     int path;                 /* DLK_PATH_AUTO; the others force one implementation (tests) */
     float softcap;            /* > 0: logits = softcap * tanhf(logits / softcap) first, as the
