@@ -176,8 +176,9 @@ DLK_DEV int lanes_below(uint64_t bal) {
 /* Of the n <= blockDim.x <= 256 entries of buf (sort keys: high word first),
  * moves those whose high word is at or below the r-th smallest high word (r <= n)
  * to the front and returns their count (r, plus any ties): the r-th high word
- * by a bitwise search on one wave, four keys a lane.  slot: two LDS words. */
-DLK_DEV int keep_best(uint64_t *buf, int n, int r, int *slot) {
+ * by a bitwise search on one wave, four keys a lane.  slot: two LDS words.  One
+ * copy out of line: its callers are rare paths (three inlined: 0.4 us on every call). */
+__device__ __noinline__ int keep_best(uint64_t *buf, int n, int r, int *slot) {
     const int t = threadIdx.x, lane = lane_id();
     const uint64_t mine = t < n ? buf[t] : ~0ull;
     if (wave_id() == 0) {
@@ -563,7 +564,7 @@ __global__ __launch_bounds__(kTopkThreads, 8) void topk_kernel(TopkParams f) {
         /* ---- 4. candidates: the entries at or above the threshold -------- */
         bool all_groups = false, over = false;
         int C = 0;
-        for (int attempt = 0; attempt < 2; attempt++) {
+        for (int attempt = 0; attempt < 4; attempt++) {
             const float te = thr > -INFINITY ? thr : -kFltMax;
             const float cte = !CAP ? te : thr > -INFINITY ? dlk_softcap_glibc(thr, p.cap) : -INFINITY;
             const int ng = misc[1];
@@ -597,8 +598,19 @@ __global__ __launch_bounds__(kTopkThreads, 8) void topk_kernel(TopkParams f) {
             __syncthreads();
             C = misc[10];
             over = (!all_groups && ng > f.grp_cap) || C > f.cand_cap;
+            if (DLK_COLD(!CAP && C > f.cand_cap && (all_groups || ng <= f.grp_cap) && f.KP <= T / 2 && attempt < 3)) {
+                /* a wave with too few groups (a last slice of some 500 to 900
+                 * entries, allowed ids in a cluster) left no threshold, and the
+                 * slice holds more than cbuf: the KP-th of any 256 entries is
+                 * one (the row fell back to the whole-row selection, 400 us) */
+                keep_best(cbuf, T, f.KP, &misc[20]);
+                thr = key_value((uint32_t)misc[20]);
+                if (t == 0) misc[10] = 0;
+                __syncthreads();
+                continue;
+            }
             if (DLK_COLD(over && !exact_done)) exact_pass();  /* the row falls back: its maximum must be exact */
-            if (DLK_HOT(over || C >= f.KP || C >= nf)) break;
+            if (DLK_HOT(over || C >= f.KP || C >= nf) || all_groups) break;
             /* fewer than KP entries reach a threshold taken from raw logits
              * (penalties lowered some of them): the exact threshold, every group */
             if (!exact_done) exact_pass();

@@ -80,3 +80,40 @@ def test_topk_many_patches(cuda, n, kw):
     if kw.get("top_k") == 9:
         w.softcap = 30.0
         run_and_check(w, 0)
+
+
+@pytest.mark.parametrize("V,k", [(131776, 60), (131761, 87), (66240, 40), (8192 * 3 + 513, 100), (65536 + 870, 112)])
+def test_topk_small_last_slice(cuda, V, k):
+    """A last slice with too few entries for a threshold from every wave and more than the candidate buffer holds,
+    and the same from a mask whose allowed ids lie in a cluster."""
+    rows = 3
+    rng = np.random.default_rng(V)
+    lg = rng.normal(0, 3, size=(rows, V)).astype(np.float32)
+    lg[1, V - 700:] += np.float32(6)
+    w = make(f"last-{V}", rows, V, seed=k, logits=lg, temperature=1.05, top_k=k, top_p=0.94, n_out=8, rep=1.2,
+             hist=[np.arange(V - 20, V), [], rng.integers(0, V, 50)])
+    run_and_check(w, 0)
+    w.mask = mask_rows(rows, V, [np.arange(5000, 5700), np.arange(9000, 9900), np.arange(V - 800, V)])
+    run_and_check(w, 0)
+
+
+def test_rows_without_workspace_under_capture(cuda):
+    """Rows of odd length captured on a stream that holds no workspace yet run on the row kernel."""
+    import torch
+    from diskllm_amd import api
+    rng = np.random.default_rng(9)
+    V = 9001
+    for kw in (dict(top_p=0.9), dict(top_k=20)):
+        w = make("capture", 3, V, seed=4, logits=rng.normal(0, 2, (3, V)).astype(np.float32), **kw)
+        want = run_and_check(w, 1)["ids"]
+        db = api.to_device(w)
+        prm = api.params_of(w)
+        g = torch.cuda.CUDAGraph()
+        torch.cuda.synchronize()
+        with torch.cuda.graph(g, stream=torch.cuda.Stream()):
+            api.sample(db, prm)
+        for _ in range(3):
+            db.reset_rng()
+            g.replay()
+            torch.cuda.synchronize()
+            np.testing.assert_array_equal(db.out_ids.cpu().numpy(), want)
