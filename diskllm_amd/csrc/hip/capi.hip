@@ -107,6 +107,13 @@ __global__ void zero_words_kernel(uint32_t *p, size_t n) {
         p[i] = 0u;
 }
 
+bool zero_words(uint32_t *p, size_t n, hipStream_t stream) {
+    unsigned blocks = (unsigned)((n + 255) / 256);
+    if (blocks > 1024) blocks = 1024;
+    hipLaunchKernelGGL(zero_words_kernel, dim3(blocks), dim3(256), 0, stream, p, n);
+    return hipGetLastError() == hipSuccess;
+}
+
 unsigned char *scratch_ptr() {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return nullptr;
@@ -127,12 +134,7 @@ bool workspace_noalloc(hipStream_t stream, int kind, size_t counters, size_t dat
     unsigned char *base = scratch_ptr();
     g_ws_err = DLK_ERR_HIP;
     if (!base) return false;
-    if (counters > 0) {
-        unsigned blocks = (unsigned)((counters + 255) / 256);
-        if (blocks > 1024) blocks = 1024;
-        hipLaunchKernelGGL(zero_words_kernel, dim3(blocks), dim3(256), 0, stream, (uint32_t *)base, counters);
-        if (hipGetLastError() != hipSuccess) return false;
-    }
+    if (counters > 0 && !zero_words((uint32_t *)base, counters, stream)) return false;
     out.counters = (uint32_t *)base;
     out.data = base + kScratchCtrWords * 4;
     return true;
@@ -168,7 +170,10 @@ bool workspace(hipStream_t stream, int kind, size_t counters, size_t data_bytes,
             w->ctr_cap = w->data_bytes = 0;
         }
         if (hipMalloc(&w->ptr, cc * 4 + db) != hipSuccess) { w->ptr = nullptr; return false; }
-        if (cc > 0 && hipMemset(w->ptr, 0, cc * 4) != hipSuccess) return false;
+        /* cleared in the order of the call's stream: one that does not wait for the
+         * null stream would start its kernels beside a hipMemset there (a first
+         * call's row barriers then timed out: 0.55 s and invalid ids) */
+        if (cc > 0 && !zero_words((uint32_t *)w->ptr, cc, stream)) return false;
         w->ctr_cap = cc;
         w->data_bytes = db;
     }

@@ -1,0 +1,43 @@
+"""The host side of dlk_sample on stand-ins for the HIP runtime (tests/native/capi_host_check.cpp): what it does with
+its workspaces around the kernel launches."""
+import os
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+BUILD = os.path.join(ROOT, "oracle", "_build")
+HIP = "/opt/rocm/bin/hipcc"
+
+
+@pytest.fixture(scope="module")
+def host():
+    os.makedirs(BUILD, exist_ok=True)
+    obj, exe = os.path.join(BUILD, "capi_host.o"), os.path.join(BUILD, "capi_host_check")
+    inc = "-I" + os.path.join(ROOT, "include")
+    subprocess.run([HIP, "--offload-arch=gfx950", "--offload-host-only", "-O1", "-std=c++17", "-fPIC", inc, "-c",
+                    os.path.join(ROOT, "diskllm_amd", "csrc", "hip", "capi.hip"), "-o", obj], check=True)
+    subprocess.run(["g++", "-O1", "-std=c++17", "-D__HIP_PLATFORM_AMD__", inc, "-I/opt/rocm/include", "-o", exe,
+                    os.path.join(ROOT, "tests", "native", "capi_host_check.cpp"), obj, "-lpthread",
+                    "-Wl,--unresolved-symbols=ignore-in-object-files"], check=True)
+
+    def run(commands):
+        r = subprocess.run([exe] + commands.split(), capture_output=True, text=True, timeout=60)
+        assert r.returncode == 0, r.stdout + r.stderr
+        return r.stdout.splitlines()
+    return run
+
+
+FULL, TOPK = "64 151936 151936 0 1.0", "64 128256 128256 40 0.8"
+
+
+@pytest.mark.parametrize("call,kernel", [(FULL, "fused"), (TOPK, "top-k")])
+def test_fresh_workspace_is_cleared_on_the_stream_of_the_call(host, call, kernel):
+    """The counters of a fresh workspace are cleared in the order of the call's own stream: a clear on the null stream
+    is not waited for by a non-blocking one, and the kernel's row barriers then count from whatever is there."""
+    out = host(f"sample {call} 7 sample {call} 7")
+    at = [i for i, line in enumerate(out) if "kernel" in line]
+    assert len(at) == 2 and all(out[i] == f"{kernel} kernel, 64 rows on stream 7" for i in at), out
+    assert out[0].startswith("malloc") and out[1] == "clear on stream 7" and at[0] == 2, out
+    assert not any("memset" in line for line in out), out
+    assert sum("clear" in line for line in out) == 1, out       # the kernels return their counters to zero
