@@ -4,18 +4,25 @@
  * all rows: under the JSON validator what a token does to a row depends only on
  * whether the row is inside a string, so one walk of its bytes gives the deepest
  * '}' and ']' it closes for either case, and each row then takes two compares.
- * Rows of the receipt validator resume their own state (grammar_scan.h) and feed
- * the token's bytes.
+ * Rows of the receipt validator are walked from their state through its transition
+ * table (grammar_table.h), four states at a time; rows of a block that share a
+ * state are walked once.
  */
 #include <hip/hip_runtime.h>
 #include <math.h>
 
-#include "grammar_scan.h"
+#include <algorithm>
+
+#include "grammar_table.h"
 
 namespace dlk {
 
 constexpr int kMaskTokens = 512;     /* a thread per token: 16 mask words, one 64-byte line per row and block */
-constexpr int kMaskRows = 64;        /* rows per block */
+constexpr int kMaskRows = 64;        /* rows per block at most (a wave's lanes, a word's bits) */
+/* Rows are split over blocks up to about this many.  16 x 151,936 JSON rows: 13.7 us
+ * at 256, 13.9 at 512, 18.3 at 1,024; 65 x 32,003: 12.8, 12.5, 17.3; 1 to 512 rows of
+ * 1,000: 8 to 9.7 at 512, up to 13.8 at 1,024 (all 64 rows to a block: 19). */
+constexpr int kMaskBlocks = 512;
 constexpr int kMaskBytes = 8192;     /* token bytes staged per block (the rest is read from memory) */
 
 /* How a row tests a token: its string fits (len <= room), closes no more braces
@@ -30,7 +37,11 @@ constexpr uint32_t kInStr = 1;       /* JSON: inside a string */
 constexpr uint32_t kEscaped = 2;     /* JSON: the previous byte is a backslash */
 constexpr uint32_t kStart = 4;       /* JSON before its first '{' or '[' */
 constexpr uint32_t kFinished = 8;    /* the EOS id's bit */
-constexpr uint32_t kScan = 16;       /* resume the row's validator byte by byte instead */
+constexpr uint32_t kWalk = 16;       /* needs the token's walk (JSON) */
+constexpr uint32_t kTable = 32;      /* a state of the receipt table */
+constexpr uint32_t kScan = 64;       /* any other: resume the row's validator byte by byte */
+constexpr int kStateShift = 8;       /* kTable: the state */
+constexpr int kFirstShift = 16;      /* kTable: the first row of the block in the same state */
 
 __device__ __forceinline__ RowTest row_test(const dlk_grammar_row &st) {
     RowTest r;
@@ -46,39 +57,60 @@ __device__ __forceinline__ RowTest row_test(const dlk_grammar_row &st) {
                s.flag <= 1) {
         r.n = s.n;
         r.m = s.m;
-        r.bits |= (s.flag ? kInStr : 0u) | (s.prev == '\\' ? kEscaped : 0u) | (s.pc == DLK_JS_WS ? kStart : 0u);
+        r.bits |= kWalk | (s.flag ? kInStr : 0u) | (s.prev == '\\' ? kEscaped : 0u) | (s.pc == DLK_JS_WS ? kStart : 0u);
     } else if (s.mode == DLK_GRAMMAR_JSON || s.mode == DLK_GRAMMAR_RECEIPT) {
-        r.bits |= kScan;
+        const int key = dlk_receipt_key(&s);
+        const uint32_t id = key >= 0 ? kReceiptTable.id[key] : 0u;
+        r.bits |= id ? kTable | id << kStateShift : kScan;
     }
     return r;
 }
 
-/* Grid (ceil(V / 512), ceil(rows / 64)): a block tests its 512 tokens against up
- * to 64 rows.  Bound by latency (offsets, then bytes, then the walk of the
+/* Grid (ceil(V / 512), ceil(rows / per)): a block tests its 512 tokens against up
+ * to `per` rows.  Bound by latency (offsets, then bytes, then the walk of the
  * block's longest token): the vocabulary is some 1.5 MB.  The token bytes are
  * contiguous, so a block stages them in LDS, eight coalesced loads a thread in
- * flight, and a walk takes four bytes per LDS read.  A walk of dependent byte
- * loads from memory per (token, row) and one atomicAdd per wave and row for the
- * counts (38,000 into one cache line) took 433 us at 16 x 151,936, this form
- * 12.6 us and the counting kernel 4.5 (kernel times under the profiler). */
+ * flight, and a walk takes four bytes per LDS read.  A walk of dependent byte loads
+ * from memory per (token, row) and one atomicAdd per wave and row for the
+ * counts (38,000 into one cache line) took 433 us at 16 x 151,936 with counts,
+ * this form 17, of which the counting kernel is some 3.  Receipt rows, 16 x
+ * 151,936 without counts: 44 us so and 112 when a block resumed its rows' scanner
+ * one row after another; 12 now where the rows share a state, 20 where all differ
+ * (65 x 1,000: 7.4, 297, 6.6 and 8.7). */
 __global__ __launch_bounds__(kMaskTokens) void grammar_mask_kernel(const uint32_t *__restrict__ off,
                                                                    const uint8_t *__restrict__ bytes, int V,
                                                                    const dlk_grammar_row *__restrict__ states,
-                                                                   int rows, int eos_id, uint32_t *mask,
+                                                                   int rows, int per, int eos_id, uint32_t *mask,
                                                                    int64_t mask_ld, float *logits, int64_t ld) {
     __shared__ uint32_t sw[kMaskBytes / 4 + 2];
     __shared__ RowTest tests[kMaskRows];
+    __shared__ uint32_t kinds;                     /* the rows' bits, or-ed */
     __shared__ uint64_t words[kMaskRows][kMaskTokens / 64];
     uint8_t *sb = (uint8_t *)sw;
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int t0 = blockIdx.x * kMaskTokens, tok = t0 + t;
-    const int r0 = blockIdx.y * kMaskRows, nr = min(kMaskRows, rows - r0);
+    const int r0 = blockIdx.y * per, nr = min(per, rows - r0);
     uint32_t b0 = 0, b1 = 0;
     if (tok < V) { b0 = off[tok]; b1 = off[tok + 1]; }
     /* the block's bytes: [lo, lo + n) staged (a token outside is read from memory) */
     const uint32_t lo = off[t0], hi = off[min(t0 + kMaskTokens, V)];
     const int n = hi > lo ? (int)min(hi - lo, (uint32_t)kMaskBytes) : 0;
-    if (t < nr) tests[t] = row_test(states[r0 + t]);
+    if (wave == 0) {
+        RowTest r = {};
+        if (lane < nr) r = row_test(states[r0 + lane]);
+        if (__ballot((r.bits & kTable) != 0)) {
+            const int id = (int)(r.bits & (kTable | 0xffu << kStateShift));
+            int first = kMaskRows;
+#pragma unroll 1
+            for (int i = nr - 1; i >= 0; i--)
+                if (id == __builtin_amdgcn_readlane(id, i)) first = i;
+            if (r.bits & kTable) r.bits |= (uint32_t)first << kFirstShift;
+        }
+        if (lane < nr) tests[lane] = r;
+        uint32_t any = 0;
+        for (uint32_t bit = kWalk; bit <= kScan; bit <<= 1) any |= __ballot((r.bits & bit) != 0) ? bit : 0u;
+        if (lane == 0) kinds = any;
+    }
     for (int i0 = 0; i0 < n; i0 += 8 * kMaskTokens) {
         uint8_t x[8];
 #pragma unroll
@@ -115,7 +147,16 @@ __global__ __launch_bounds__(kMaskTokens) void grammar_mask_kernel(const uint32_
     int len = 0, lead = 0, par = 0;                /* lead: 0 whitespace so far, 1 then '{' or '[', 2 anything else */
     int db0 = 0, db1 = 0, dk0 = 0, dk1 = 0, nb0 = 0, nb1 = 0, nk0 = 0, nk1 = 0;
     bool quote1 = false, esc = false, ended = false;   /* the first byte is '"'; the last was a backslash */
-    for (uint32_t i = 0; i < cap && !ended; i += 4) {
+    const uint32_t any = kinds;
+    if (!(any & kWalk)) {
+        /* (no JSON row: the string's length is enough) */
+        for (uint32_t i = 0; i < cap && !ended; i += 4) {
+            const uint32_t x = word_at(i);         /* (bytes past the token's end are 0 too) */
+            const uint32_t zero = (x - 0x01010101u) & ~x & 0x80808080u;
+            ended = zero != 0;
+            len += ended ? __builtin_ctz(zero) >> 3 : 4;
+        }
+    } else for (uint32_t i = 0; i < cap && !ended; i += 4) {
         const uint32_t x = word_at(i);
         if (i == 0) quote1 = (x & 0xffu) == '"';
 #pragma unroll
@@ -133,41 +174,59 @@ __global__ __launch_bounds__(kMaskTokens) void grammar_mask_kernel(const uint32_
         }
     }
 
-    bool scan = false;
     const int fit = len > 0 ? len : 0x7fffffff;    /* the empty string is never allowed (:294-298) */
     const uint32_t flip = quote1 ? kEscaped : 0u;
+    uint64_t fed = 0;                              /* bit r: the string passes the validator in row r's state */
+    if (any & kTable) {
+        /* the block's states four at a time (the same in every thread) */
+        for (int r = 0; r < nr;) {
+            uint32_t at[4] = {};
+            int rows4[4], n4 = 0;
+            for (; r < nr && n4 < 4; r++) {
+                const uint32_t bits = tests[r].bits;
+                if (!(bits & kTable) || (int)(bits >> kFirstShift) != r) continue;
+#pragma unroll
+                for (int q = 0; q < 4; q++)
+                    if (q == n4) { at[q] = (bits >> kStateShift) & 0xffu; rows4[q] = r; }
+                n4++;
+            }
+            uint32_t x = 0;
+            for (int i = 0; i < len && (at[0] | at[1] | at[2] | at[3]); i++) {
+                if ((i & 3) == 0) x = word_at((uint32_t)i);
+                const uint32_t c = kReceiptTable.cls[x & 0xffu];
+#pragma unroll
+                for (int q = 0; q < 4; q++) at[q] = kReceiptTable.next[at[q]][c];
+                x >>= 8;
+            }
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+                if (q < n4 && at[q]) fed |= 1ull << rows4[q];
+        }
+    }
+    if (any & kScan) {
+        for (int r = 0; r < nr; r++) {
+            if (!(tests[r].bits & kScan)) continue;
+            dlk_scan_state s = states[r0 + r].scan;
+            uint32_t x = 0;
+            for (int i = 0; i < len && dlk_scan_ok(&s); i++) {
+                if ((i & 3) == 0) x = word_at((uint32_t)i);
+                dlk_scan_step(&s, (uint8_t)x);
+                x >>= 8;
+            }
+            if (dlk_scan_ok(&s)) fed |= 1ull << r;
+        }
+    }
     for (int r = 0; r < nr; r++) {
         const RowTest R = tests[r];
         /* an escaped first quote does not toggle: the other case's walk from there on */
         const bool in = ((R.bits & kInStr) != 0) != ((R.bits & flip) != 0);
         bool ok = fit <= R.room && len > 0 && R.n >= (in ? nb1 : nb0) && R.m >= (in ? nk1 : nk0) &&
                   !((R.bits & kStart) && lead == 2);
+        if (R.bits & (kTable | kScan)) ok = ok && ((fed >> (R.bits & kTable ? R.bits >> kFirstShift : r)) & 1u);
         if (tok == eos_id) ok = (R.bits & kFinished) != 0;               /* :285-291 */
         ok = ok && tok < V;
-        scan = scan || (R.bits & kScan);
         const uint64_t bal = __ballot(ok);
         if (lane == 0) words[r][wave] = bal;
-    }
-    if (scan) {
-        /* (the same answer in every thread of the block) */
-        for (int r = 0; r < nr; r++) {
-            const RowTest R = tests[r];
-            if (!(R.bits & kScan)) continue;
-            bool ok = len > 0 && len <= R.room && tok < V;
-            if (ok) {
-                dlk_scan_state s = states[r0 + r].scan;
-                uint32_t x = 0;
-                for (int i = 0; i < len && dlk_scan_ok(&s); i++) {
-                    if ((i & 3) == 0) x = word_at((uint32_t)i);
-                    dlk_scan_step(&s, (uint8_t)x);
-                    x >>= 8;
-                }
-                ok = dlk_scan_ok(&s);
-            }
-            if (tok == eos_id && tok < V) ok = (R.bits & kFinished) != 0;
-            const uint64_t bal = __ballot(ok);
-            if (lane == 0) words[r][wave] = bal;
-        }
     }
     __syncthreads();
     if (logits && tok < V)
@@ -233,10 +292,14 @@ extern "C" int dlk_grammar_mask(const uint32_t *off, const uint8_t *bytes, int v
     using namespace dlk;
     if (!off || !bytes || !states || !mask || vocab <= 0 || rows <= 0 || rows > 65535) return DLK_ERR_INVALID;
     if (mask_ld < (vocab + 31) / 32 || (logits && ld < vocab)) return DLK_ERR_INVALID;
-    hipLaunchKernelGGL(grammar_mask_kernel,
-                       dim3((vocab + kMaskTokens - 1) / kMaskTokens, (rows + kMaskRows - 1) / kMaskRows),
-                       dim3(kMaskTokens), 0, stream, off, bytes, vocab, states, rows, eos_id, mask, mask_ld, logits,
-                       ld);
+    /* rows per block: as many as leave about kMaskBlocks blocks (each walks its tokens
+     * again for its rows), between one and kMaskRows */
+    const int gx = (vocab + kMaskTokens - 1) / kMaskTokens;
+    int gy = std::max((rows + kMaskRows - 1) / kMaskRows, std::min(rows, (kMaskBlocks + gx - 1) / gx));
+    const int per = (rows + gy - 1) / gy;
+    gy = (rows + per - 1) / per;
+    hipLaunchKernelGGL(grammar_mask_kernel, dim3(gx, gy), dim3(kMaskTokens), 0, stream, off, bytes, vocab, states, rows,
+                       per, eos_id, mask, mask_ld, logits, ld);
     if (valid)
         hipLaunchKernelGGL(mask_count_kernel, dim3(rows), dim3(1024), 0, stream, mask, mask_ld, (vocab + 31) / 32,
                            valid);

@@ -25,7 +25,9 @@
 #include "../../../include/diskllm_amd.h"
 
 #if defined(__HIPCC__)
-#define DLK_GHD __host__ __device__ inline
+#define DLK_GHD __host__ __device__ constexpr inline
+#elif defined(__cplusplus)
+#define DLK_GHD constexpr inline
 #else
 #define DLK_GHD static inline
 #endif

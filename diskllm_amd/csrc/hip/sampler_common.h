@@ -156,7 +156,7 @@ __device__ __forceinline__ void rank_sort_distinct(K *a, int n) {
 #pragma unroll
             for (int u = 0; u < 8; u++) o[u] = a[j + (u << sh)];
 #pragma unroll
-            for (int u = 0; u < 8; u++) r += (j + (u << sh) < n) & (o[u] < key) ? 1 : 0;
+            for (int u = 0; u < 8; u++) r += ((j + (u << sh) < n) & (o[u] < key)) ? 1 : 0;
         }
     }
     /* the neighbours' counts (quad permutations: swap pairs, swap halves) */

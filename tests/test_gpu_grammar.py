@@ -69,3 +69,75 @@ def test_grammar_mask_shapes(cuda, V, rows, longest):
         assert valid[r] == n, pick
         np.testing.assert_array_equal(got[r, :V], np.where(want, logits[r, :V], -np.inf))
         np.testing.assert_array_equal(got[r, V:], logits[r, V:])
+
+
+RECEIPT = b'{"bbox_2d":[1, 2,3,4], "text_content": "a\\b"}'
+
+
+def step_us(torch, L, V, mode, bufs, calls=20):
+    """Microseconds of one mask call, the shortest of five runs of `calls`."""
+    off, data = token_table(np.random.default_rng(V), V, 16)
+    states = (_lib.GrammarRow * len(bufs))()
+    for s, buf in zip(states, bufs):
+        L.dlk_grammar_row_init(C.byref(s), mode)
+        L.dlk_grammar_row_feed(C.byref(s), buf, len(buf))
+    d = [torch.from_numpy(x).cuda() for x in (off.view(np.int32), data, np.frombuffer(bytes(states), np.uint8).copy())]
+    W = (V + 31) // 32
+    mask = torch.zeros((len(bufs), W), dtype=torch.int32, device="cuda")
+    best = np.inf
+    for _ in range(6):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        a.record()
+        for _ in range(calls):
+            L.dlk_grammar_mask(d[0].data_ptr(), d[1].data_ptr(), V, d[2].data_ptr(), len(bufs), V - 1, mask.data_ptr(), W,
+                               None, 0, None, torch.cuda.current_stream().cuda_stream)
+        b.record()
+        b.synchronize()
+        best = min(best, a.elapsed_time(b) * 1e3 / calls)
+    return best
+
+
+def test_rows_are_not_taken_one_after_another(cuda):
+    """Receipt rows cost about what JSON rows do, whether they share a state or not, and 65 rows of a small vocabulary
+    about what one does (a block that took them in turn made them 15 and 2.3 times as long)."""
+    L = _lib.lib()
+    one = step_us(cuda, L, 1000, 1, [b"{"])
+    many = step_us(cuda, L, 1000, 1, [b"{"] * 65)
+    same = step_us(cuda, L, 1000, 2, [b""] * 65)
+    unlike = step_us(cuda, L, 1000, 2, [RECEIPT[:i % len(RECEIPT)] for i in range(65)])
+    print(f"[case] 1000 tokens: one row {one:.1f} us, 65 {many:.1f}, 65 receipt rows {same:.1f} and {unlike:.1f}", flush=True)
+    assert many < 1.6 * one and max(same, unlike) < 2.5 * many
+
+
+@pytest.mark.parametrize("V,rows", [(700, 70), (1536, 9)])
+def test_receipt_states(cuda, V, rows):
+    """Every position of a receipt, several to a block, states that no buffer leads to (they are scanned byte by
+    byte), and a validator that has rejected."""
+    import torch
+    L = _lib.lib()
+    rng = np.random.default_rng(V)
+    off, data = token_table(rng, V, 60)
+    states = (_lib.GrammarRow * rows)()
+    for i, s in enumerate(states):
+        L.dlk_grammar_row_init(C.byref(s), 2)
+        buf = RECEIPT[:i % (len(RECEIPT) + 1)] + (b"}" if i % 19 == 18 else b"")
+        L.dlk_grammar_row_feed(C.byref(s), buf, len(buf))
+        if i % 7 == 6:
+            s.scan.flag ^= 1                                     # (a digit or none, where no position has it so)
+        if i % 11 == 10:
+            s.scan.m = 3
+            s.scan.n = 9 if s.scan.pc == 2 else s.scan.n
+    d = [torch.from_numpy(x).cuda() for x in (off.view(np.int32), data, np.frombuffer(bytes(states), np.uint8).copy())]
+    W = (V + 31) // 32
+    mask = torch.zeros((rows, W), dtype=torch.int32, device="cuda")
+    assert L.dlk_grammar_mask(d[0].data_ptr(), d[1].data_ptr(), V, d[2].data_ptr(), rows, -1, mask.data_ptr(), W, None, 0,
+                              None, torch.cuda.current_stream().cuda_stream) == 0
+    torch.cuda.synchronize()
+    bits = mask.cpu().numpy().view(np.uint32)
+    for r in range(rows):
+        for t in range(V):
+            tok = bytes(data[off[t]:off[t + 1]]).split(b"\0")[0]
+            s = _lib.GrammarRow()
+            C.memmove(C.byref(s), C.byref(states[r]), C.sizeof(s))
+            L.dlk_grammar_row_feed(C.byref(s), tok, len(tok))    # (the scanner, on the host)
+            assert ((bits[r, t >> 5] >> (t & 31)) & 1) == (len(tok) > 0 and s.scan.pc != 255), (r, t, tok)
