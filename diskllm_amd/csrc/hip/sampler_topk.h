@@ -11,7 +11,7 @@ namespace dlk {
 constexpr int kTopkThreads = 256;
 constexpr int kSelWords = 260;              /* radix-select histogram (256) + broadcast words */
 constexpr int kMergePerThread = 8;          /* merge: candidates per thread (G * KP <= 2048) */
-constexpr int kTopkGroupCap = 1024;         /* listed 16-byte groups per slice at most (more: the row falls back) */
+constexpr int kTopkGroupCap = 1024;         /* listed 16-byte groups per slice at most (more: select_slice) */
 constexpr int kTopkMaxG = 64;               /* workgroups per row */
 constexpr int kTopkMaxS = 65536;            /* slice length */
 constexpr int kTopkMaxK = 496;              /* four waves' thresholds need KP = k + 16 <= 4 * 128 */
@@ -23,7 +23,8 @@ struct TopkSlot {
     uint32_t argmax;     /* its lowest index */
     uint32_t nfin;       /* finite entries in the slice */
     uint32_t kept;       /* candidates published */
-    uint32_t complete;   /* 1: every finite entry published; 0: partial; 0xffffffff: overflow */
+    uint32_t complete;   /* bit 0: every finite entry published; bit 1: those published are the slice's
+                            best by (value desc, index asc) */
     uint32_t last_key;   /* desc key of the last published candidate */
     uint32_t first_nan;  /* bit 0 (slice 0): prepared logit 0 is NaN; bit 1: NaN or +inf in the slice */
     uint32_t pad;

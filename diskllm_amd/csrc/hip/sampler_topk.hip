@@ -210,6 +210,45 @@ __device__ __noinline__ int keep_best(uint64_t *buf, int n, int r, int *slot) {
     return slot[1];
 }
 
+/* An upper bound on the r-th smallest of the n <= 4 * kTopkThreads entries of buf
+ * (value key high, index low; all unlike), at most 16 places past it: eight bits a
+ * pass through a histogram.  hist: kSelWords LDS words.  Out of line and small: what
+ * it does not touch stays in its caller's registers (a selection over the slice in
+ * one function, 40 registers, made the kernel spill and every call 4 us slower). */
+__device__ __noinline__ uint64_t rth_entry(const uint64_t *buf, int n, int r, int *hist) {
+    const int t = threadIdx.x, lane = lane_id();
+    uint64_t pre = 0;
+#pragma unroll 1
+    for (int shift = 56;; shift -= 8) {
+        hist[t] = 0;
+        __syncthreads();
+#pragma unroll 1
+        for (int i = t; i < n; i += kTopkThreads) {
+            const uint64_t x = buf[i];
+            if (shift == 56 || x >> (shift + 8) == pre) atomicAdd(&hist[(int)(x >> shift) & 255], 1);
+        }
+        __syncthreads();
+        if (wave_id() == 0) {
+            int mine = 0;
+            for (int i = 0; i < 4; i++) mine += hist[4 * lane + i];
+            int before = (int)wave_scan_sat_u32((uint32_t)mine, 0x10000u) - mine;
+            if (lane == first_lane(ballot(before + mine >= r))) {
+                int i = 4 * lane;
+                while (before + hist[i] < r) before += hist[i++];
+                hist[256] = i;
+                hist[257] = before;
+                hist[258] = hist[i];
+            }
+        }
+        __syncthreads();
+        const int bin = hist[256], before = hist[257], in = hist[258];
+        __syncthreads();
+        pre = pre << 8 | (uint32_t)bin;
+        r -= before;
+        if (in - r <= 16 || shift == 0) return (pre << shift) | ((1ull << shift) - 1);
+    }
+}
+
 /* The slice of a row that one workgroup streams: groups of four elements at
  * s0 + 4 * (t + j * T), j = 0 .. S/(4T) - 1, in batches of four groups per thread
  * with the next batch's loads in flight.
@@ -561,19 +600,26 @@ __global__ __launch_bounds__(kTopkThreads, 8) void topk_kernel(TopkParams f) {
             exact_done = true;
         };
         if (DLK_COLD(misc[8])) exact_pass();
-        /* ---- 4. candidates: the entries at or above the threshold -------- */
-        bool all_groups = false, over = false;
-        int C = 0;
-        for (int attempt = 0; attempt < 4; attempt++) {
+        /* ---- 4. candidates: the entries at or above the threshold --------
+         * Where they are more than cbuf holds (a wave with too few groups for a
+         * threshold: a last slice of some 500 to 900 entries, allowed ids in a
+         * cluster; large k; equal logits) the KP-th of those in cbuf, by (value
+         * desc, index asc), is a bound: they are collected again up to it, at most
+         * half as many each time where their order is no matter.  Turned about each
+         * time, so that a sorted slice does not fill cbuf with its worst first.  (The
+         * row fell back to one workgroup's selection over all of it: 300 x 50,257 with
+         * k 200 383 us, 91 so; 2 x 131,776 with k 60 and a cap 1,650 and 26; 64 x
+         * 50,257 equal logits with k 40 570 and 85; 32 x 262,144 with k 300 1,446 and
+         * 137.)  The first pass has a loop of its own: sharing this one made every
+         * call 0.6 us slower. */
+        const int ng = misc[1];
+        {
             const float te = thr > -INFINITY ? thr : -kFltMax;
             const float cte = !CAP ? te : thr > -INFINITY ? dlk_softcap_glibc(thr, p.cap) : -INFINITY;
-            const int ng = misc[1];
-            const int lim = all_groups ? f.S / 4 : min(ng, f.grp_cap);
-            for (int k2 = t; k2 < lim; k2 += T) {
+            for (int k2 = t; k2 < min(ng, f.grp_cap); k2 += T) {
                 /* (a listed group below the final threshold holds no candidate) */
-                if (!all_groups && !(gmx[k2] >= te)) continue;
-                const int i0 = all_groups ? s0 + 4 * k2 : (int)grp[k2];
-                if (i0 >= s1) continue;
+                if (!(gmx[k2] >= te)) continue;
+                const int i0 = (int)grp[k2];
                 const float4 v = load_group(lg, i0, s1);
                 const uint32_t live = group_live<GREEDY>(mk ? mk[i0 >> 5] >> (i0 & 31) : 0xFu, gbits, pt, i0, s0, s1);
                 const float e[4] = {v.x, v.y, v.z, v.w};
@@ -595,30 +641,73 @@ __global__ __launch_bounds__(kTopkThreads, 8) void topk_kernel(TopkParams f) {
                     if (at < f.cand_cap) cbuf[at] = ((uint64_t)desc_key(y) << 32) | (uint32_t)id;
                 }
             }
-            __syncthreads();
-            C = misc[10];
-            over = (!all_groups && ng > f.grp_cap) || C > f.cand_cap;
-            if (DLK_COLD(!CAP && C > f.cand_cap && (all_groups || ng <= f.grp_cap) && f.KP <= T / 2 && attempt < 3)) {
-                /* a wave with too few groups (a last slice of some 500 to 900
-                 * entries, allowed ids in a cluster) left no threshold, and the
-                 * slice holds more than cbuf: the KP-th of any 256 entries is
-                 * one (the row fell back to the whole-row selection, 400 us) */
-                keep_best(cbuf, T, f.KP, &misc[20]);
-                thr = key_value((uint32_t)misc[20]);
+        }
+        __syncthreads();
+        int C = misc[10];
+        bool over = ng > f.grp_cap || C > f.cand_cap, placed = false;   /* placed: cbuf holds final values */
+        if (DLK_COLD(over || (C < f.KP && C < nf))) {
+            uint64_t bound = ~0ull;
+            bool all_groups = false, exact_thr = false;
+#pragma unroll 1
+            for (int attempt = 1; attempt < 8 && !(over && irr); attempt++) {
+                if (!over) {
+                    /* fewer than KP entries reach a threshold taken from raw logits
+                     * (penalties lowered some of them): the exact threshold, every group */
+                    if (!exact_done) exact_pass();
+                    thr = ethr;
+                    exact_thr = true;
+                    all_groups = true;
+                } else {
+                    if (C > f.cand_cap && (placed || !CAP)) bound = rth_entry(cbuf, f.cand_cap, f.KP, selh);
+                    placed = true;
+                    all_groups = all_groups || ng > f.grp_cap;
+                }
+                __syncthreads();
                 if (t == 0) misc[10] = 0;
                 __syncthreads();
-                continue;
+                const float te = thr > -INFINITY ? thr : -kFltMax;
+                const float cte = !CAP ? te : thr > -INFINITY ? dlk_softcap_glibc(thr, p.cap) : -INFINITY;
+                /* (a reservation per wave: there may be thousands) */
+                auto push = [&](bool on, float y, int id) {
+                    const uint64_t x = ((uint64_t)desc_key(y) << 32) | (uint32_t)id;
+                    const uint64_t b2 = ballot(on && x <= bound);
+                    if (!b2) return;
+                    int at = 0;
+                    if (lane == 0) at = atomicAdd(&misc[10], (int)__popcll(b2));
+                    at = __builtin_amdgcn_readfirstlane(at) + lanes_below(b2);
+                    if (((b2 >> lane) & 1ull) && at < f.cand_cap) cbuf[at] = x;
+                };
+                const int lim = all_groups ? f.S / 4 : ng;
+#pragma unroll 1
+                for (int k1 = 0; k1 < lim; k1 += T) {
+                    const int k2 = attempt & 1 ? lim - 1 - (k1 + t) : k1 + t;
+                    const bool in = k2 >= 0 && k2 < lim && (all_groups || gmx[k2] >= te);
+                    const int i0 = !in ? s1 : all_groups ? s0 + 4 * k2 : (int)grp[k2];
+                    const float4 v = load_group(lg, i0, s1);
+                    const uint32_t live =
+                        i0 < s1 ? group_live<GREEDY>(mk ? mk[i0 >> 5] >> (i0 & 31) : 0xFu, gbits, pt, i0, s0, s1) : 0u;
+#pragma unroll 1
+                    for (int c = 0; c < 4; c++) {
+                        float y = c == 0 ? v.x : c == 1 ? v.y : c == 2 ? v.z : v.w;
+                        if (CAP) y = fminf(fmaxf(y, -kFltMax), kFltMax);
+                        const bool on = ((live >> c) & 1u) && y >= te;
+                        if (CAP && placed && on) y = dlk_softcap_glibc(y, p.cap);
+                        push(on, y, i0 + c);
+                    }
+                }
+#pragma unroll 1
+                for (int k1 = 0; k1 < npt; k1 += T) {
+                    const int id = k1 + t < npt ? pt.key[k1 + t] : -1;
+                    const float y = id >= 0 ? pt.value(k1 + t) : -INFINITY;
+                    push(y > -INFINITY && y >= cte, y, id);
+                }
+                __syncthreads();
+                C = misc[10];
+                over = C > f.cand_cap;
+                if (!over && (C >= f.KP || C >= nf || exact_thr)) break;
             }
-            if (DLK_COLD(over && !exact_done)) exact_pass();  /* the row falls back: its maximum must be exact */
-            if (DLK_HOT(over || C >= f.KP || C >= nf) || all_groups) break;
-            /* fewer than KP entries reach a threshold taken from raw logits
-             * (penalties lowered some of them): the exact threshold, every group */
-            if (!exact_done) exact_pass();
-            thr = ethr;
-            all_groups = true;
-            if (t == 0) misc[10] = 0;
-            __syncthreads();
         }
+        if (DLK_COLD(over && !exact_done)) exact_pass();   /* the row falls back: its maximum must be exact */
         bm = -INFINITY;
         if (exact_done) {
             bm = smax;
@@ -626,9 +715,9 @@ __global__ __launch_bounds__(kTopkThreads, 8) void topk_kernel(TopkParams f) {
             bm = fmaxf(bm, pmv);
         }
         if (over) {
-            complete = -1;                         /* overflow: the merge falls back */
+            complete = 4;                          /* overflow: the merge falls back */
         } else if (C > 0) {
-            if (CAP) {
+            if (CAP && !placed) {
                 /* cap the streamed entries (the patches' values are capped already) */
                 for (int i = t; i < C; i += T) {
                     const uint64_t e = cbuf[i];
@@ -657,8 +746,10 @@ __global__ __launch_bounds__(kTopkThreads, 8) void topk_kernel(TopkParams f) {
              * slice maximum */
             if (!exact_done) bm = key_value((uint32_t)(cbuf[0] >> 32));
             kept = min(f.KP, n);
-            complete = kept == nf ? 1 : 0;
             last_key = (uint32_t)(cbuf[kept - 1] >> 32);
+            /* (under CAP an entry that the raw threshold left out may share its value) */
+            const bool in_order = !CAP || last_key < desc_key(thr > -INFINITY ? dlk_softcap_glibc(thr, p.cap) : -INFINITY);
+            complete = (kept == nf ? 1 : 0) | (in_order ? 2 : 0);
             uint64_t *cands = f.cands + ((int64_t)row * G + g) * f.KP;
             for (int j = t; j < kept; j += T) pub64(&cands[j], cbuf[j]);
         } else {
@@ -725,7 +816,7 @@ __global__ __launch_bounds__(kTopkThreads, 8) void topk_kernel(TopkParams f) {
         first_nan = (int)(sw[192 + lane] & 1u);
         irregular = (int)(sw[192 + lane] & 2u);
         total = (int)sk[3 * lane];
-        overflow = (int)sk[3 * lane + 1] == -1;
+        overflow = (sk[3 * lane + 1] & 4u) != 0;
     }
     if (GREEDY) {
         for (int m2 = 32; m2 >= 1; m2 >>= 1) {
@@ -848,6 +939,32 @@ __global__ __launch_bounds__(kTopkThreads, 8) void topk_kernel(TopkParams f) {
         }
         __syncthreads();
         int nsort = misc[46];
+        /* more than buf holds (equal s at the bound, a short list among few): the
+         * k-th of those in buf, by (s desc, index asc), is a bound; gathered again up
+         * to it from the lists, read anew so that no registers hold them until here */
+#pragma unroll 1
+        for (int attempt = 0; DLK_COLD(nsort > f.buf_cap) && attempt < 6; attempt++) {
+            const uint64_t bound = rth_entry(buf, f.buf_cap, k, selh);
+            __syncthreads();
+            if (t == 0) misc[46] = 0;
+            __syncthreads();
+#pragma unroll 1
+            for (int i0 = 0; i0 < GK; i0 += T) {
+                const int i = attempt & 1 ? i0 + t : GK - 1 - (i0 + t), h2 = i / KP;
+                uint64_t x = ~0ull;
+                if (i >= 0 && i < GK && i - h2 * KP < (int)sk[3 * h2]) {
+                    const uint64_t e = get64(&crow[i]);
+                    x = ((uint64_t)desc_key((key_value((uint32_t)(e >> 32)) - M) * R.inv_t) << 32) | (uint32_t)e;
+                }
+                const uint64_t b2 = ballot(x <= bound);
+                int at = 0;
+                if (lane == 0 && b2) at = atomicAdd(&misc[46], (int)__popcll(b2));
+                at = __builtin_amdgcn_readfirstlane(at) + lanes_below(b2);
+                if (((b2 >> lane) & 1ull) && at < f.buf_cap) buf[at] = x;
+            }
+            __syncthreads();
+            nsort = misc[46];
+        }
         if (DLK_COLD(nsort > f.buf_cap)) {
             ok = false;
         } else {
@@ -866,11 +983,26 @@ __global__ __launch_bounds__(kTopkThreads, 8) void topk_kernel(TopkParams f) {
                 /* certify: every slice that kept only part of its finite
                  * elements must have its last kept candidate strictly below
                  * the k-th s (one wave: G <= 64) */
-                const uint32_t kth = (uint32_t)(buf[k - 1] >> 32);
+                const uint32_t kth = (uint32_t)(buf[k - 1] >> 32), kid = (uint32_t)buf[k - 1];
                 bool bad = false;
-                if (lane < G && (int)sk[3 * lane + 1] != 1)
+                if (lane < G && !(sk[3 * lane + 1] & 1u))
                     bad = !(desc_key((key_value(sk[3 * lane + 2]) - M) * R.inv_t) > kth);
-                if (ballot(bad)) ok = false;
+                if (DLK_COLD(ballot(bad) != 0)) {
+                    /* or, at the k-th s itself, leave out nothing before the k-th
+                     * entry's index: a slice that starts past it, or whose last kept
+                     * entry is at or past it, the entries it left out being of the
+                     * same logit and behind that one or of a lower logit that is
+                     * below the k-th s */
+                    if (bad && sk[3 * lane] > 0u) {
+                        const uint32_t lk = sk[3 * lane + 2], id = (uint32_t)get64(&crow[lane * KP + (int)sk[3 * lane] - 1]);
+                        const uint32_t below = lk == desc_key(0.0f) ? lk + 2 : lk + 1;   /* (-0 is 0) */
+                        bad = desc_key((key_value(lk) - M) * R.inv_t) != kth ||
+                              !((uint32_t)(lane * f.S) > kid ||
+                                ((sk[3 * lane + 1] & 2u) && id >= kid &&
+                                 desc_key((key_value(below) - M) * R.inv_t) > kth));
+                    }
+                    if (ballot(bad)) ok = false;
+                }
             } else {
                 /* fewer finite entries than k: all of them plus the first k-NF
                  * entries that are -inf, in index order */

@@ -97,6 +97,64 @@ def test_topk_small_last_slice(cuda, V, k):
     run_and_check(w, 0)
 
 
+@pytest.mark.parametrize("rows,V,k", [(3, 131776, 113), (2, 66240, 300), (5, 50257, 200), (2, 131072 + 600, 211),
+                                      (3, 8192 * 3 + 513, 112), (300, 20481, 130)])
+@pytest.mark.parametrize("cap", [0.0, 30.0])
+def test_topk_more_candidates_than_the_buffer_holds(cuda, rows, V, k, cap):
+    """Slices that leave too many candidates whatever their threshold: large k, short last slices, allowed ids in a
+    cluster, sorted rows, equal logits (one value, two, quantised), the best ids penalised, with and without a cap."""
+    rng = np.random.default_rng(V + k)
+    lg = rng.normal(0, 3, size=(rows, V)).astype(np.float32)
+    for r in range(rows):
+        kind = r % 6
+        if kind == 1:
+            lg[r] = np.round(lg[r] * 4) / 4                  # (as logits rounded to fewer bits are)
+        elif kind == 2:
+            lg[r] = np.sort(lg[r])[::(-1) ** (r // 6)]
+        elif kind == 3:
+            lg[r] = np.float32(r % 2)                        # all equal
+        elif kind == 4:
+            lg[r] = np.where(rng.random(V) < 0.3, np.float32(2.5), np.float32(-1))
+    hist = [np.argsort(-lg[r], kind="stable")[:40] if r % 2 else [] for r in range(rows)]
+    w = make(f"over-{V}-{k}-{cap}", rows, V, seed=k, logits=lg, temperature=1.1, top_k=k, top_p=0.97, n_out=8, rep=1.2,
+             hist=hist)
+    w.softcap = cap
+    run_and_check(w, 0)
+    allowed = [np.arange(5000, 5000 + k + 900), np.arange(V - 1200, V), np.arange(0, V, 3)]
+    w.mask = mask_rows(rows, V, [allowed[r % 3] for r in range(rows)])
+    run_and_check(w, 0)
+
+
+def call_us(torch, w, path):
+    from diskllm_amd import api
+    db = api.to_device(w)
+    f = api.sampler(db, api.params_of(w, path=path))
+    best = np.inf
+    for _ in range(5):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        a.record()
+        for _ in range(5):
+            f()
+        b.record()
+        b.synchronize()
+        best = min(best, a.elapsed_time(b) * 1e3 / 5)
+    return best
+
+
+@pytest.mark.parametrize("rows,V,k,flat", [(300, 50257, 200, False), (64, 50257, 150, False), (64, 50257, 40, True),
+                                           (8, 151937, 150, False)])
+def test_topk_is_not_behind_the_row_kernel(cuda, rows, V, k, flat):
+    """Rows of odd length took the row kernel before the fused one did: large k and equal logits must not cost more
+    there (383 us against 229, 213 against 85, 570 against 186, while such slices fell back to one workgroup's
+    selection over the whole row)."""
+    rng = np.random.default_rng(k)
+    lg = np.zeros((rows, V), np.float32) if flat else rng.normal(0, 2.5, size=(rows, V)).astype(np.float32)
+    w = make(f"time-{rows}-{V}-{k}", rows, V, seed=k, logits=lg, top_k=k, temperature=0.8)
+    auto, row = call_us(cuda, w, 0), call_us(cuda, w, 1)
+    print(f"[case] {rows} x {V} k {k}: {auto:.1f} us, row kernel {row:.1f}", flush=True)
+    assert auto < 1.1 * row
+
+
 def test_rows_without_workspace_under_capture(cuda):
     """Rows of odd length captured on a stream that holds no workspace yet run on the row kernel."""
     import torch
