@@ -209,6 +209,34 @@ dlk::RowParams rows_from(const dlk::RowParams &p, int r0) {
  * and holds none yet) they run on the row kernel, which needs none. */
 bool row_kernel_instead(const dlk::RowParams &p) { return ((uintptr_t)p.logits & 15) != 0 || (p.ld & 3) != 0; }
 
+/* Where the row kernel (1,024 threads to a row) is the faster one for a top-k or
+ * greedy call: its rows in one round of the CUs, and
+ *  - greedy over a short row, whose one pass costs less than publishing and merging
+ *    slices: no history, up to 12,288 ids (1 x 2,001: 4.9 us against 7.3; 64 x 8,193:
+ *    6.6 against 8.0; 64 x 12,288: 7.3 against 7.8, 64 x 16,385: 8.1 against 8.5),
+ *    and a history of up to 256, up to 4,608 ids (64 x 4,100 with 128 ids: 15 against
+ *    25; 64 x 6,144: 16.4 against 15.4);
+ *  - k above 112 (up to there the fused kernel is never behind, 64 x 1,001 with k 100:
+ *    32 against 33), where the candidates' pipeline is most of a call and 256 threads
+ *    are slow at it: rows shorter than 160 (k - 75) where nothing but the logits goes
+ *    into them (64 x 10,000 with k 150: 48 against 55, 64 x 12,288 49 against 43;
+ *    64 x 16,385 with k 300: 58 against 75, 3 x 66,240 140 against 94), any row past
+ *    k 400 (8 x 151,936 with k 496: 195 against 254); 50 (k - 120) where each of its
+ *    passes applies penalties, a mask or the soft-cap again (64 x 8,193 with 128 ids
+ *    and k 300: 75 against 86, 64 x 12,288 85 against 72).  In two rounds only past
+ *    k 400 and up to 20,480 ids (300 x 16,385 with k 496: 117 against 134; 300 x
+ *    8,193 with k 300: 90 both). */
+bool row_kernel_first(const dlk::RowParams &p, int rows, int vocab, int k, int n_cu) {
+    const bool plain = !p.hist_off && !p.mask && !(p.cap > 0.0f);
+    if (rows > 2 * n_cu) return false;
+    if (p.greedy)
+        return rows <= n_cu && !p.mask &&
+               (p.hist_off ? p.plan.hcap <= 256 && vocab <= 4608 : vocab <= 12288);
+    if (k <= 112) return false;
+    if (rows > n_cu) return plain && k > 400 && vocab <= 20480;
+    return plain ? k > 400 || vocab < 160 * (k - 75) : vocab < 50 * (k - 120);
+}
+
 /* Single-pass top-k path (sampler_topk.hip): returns DLK_OK, or 1 when the
  * configuration is outside its range (the caller then uses the row kernel). */
 int launch_topk(dlk::RowParams &p, int rows, int vocab, hipStream_t stream) {
@@ -248,6 +276,7 @@ int launch_topk(dlk::RowParams &p, int rows, int vocab, hipStream_t stream) {
     if (dev < 0 || dev >= 64) return DLK_ERR_HIP;
     if (!n_cu[dev] && hipDeviceGetAttribute(&n_cu[dev], hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
         return DLK_ERR_HIP;
+    if (row_kernel_first(p, rows, vocab, k, n_cu[dev])) return 1;
     /* occupancy per (device, kind, LDS): a fixed table, so that no call
      * allocates host memory either (past its size a query is simply repeated) */
     struct Occ { int dev, kind; size_t lds; int n; };

@@ -72,13 +72,16 @@ int dlk_launch_long_history_fixup(int, const int32_t *, const uint64_t *, uint64
 int dlk_launch_prepare_rows(const float *, int64_t, float *, int64_t, int, int, const uint32_t *, int64_t, const int32_t *, float, hipStream_t) { printf("prepare\n"); return launched(); }
 }
 
-/* commands: "memory N", "resident N", "capture 0|1", "release S", "sample ROWS VOCAB LD TOPK TEMPERATURE STREAM" */
+/* commands: "memory N", "resident N", "capture 0|1", "release S", "history N" (longest history of the next calls),
+ * "sample ROWS VOCAB LD TOPK TEMPERATURE STREAM" */
 int main(int argc, char **argv) {
+    int history = 0;
     for (int i = 1; i < argc;) {
         const std::string c = argv[i++];
         if (c == "memory") g_memory = strtoull(argv[i++], 0, 0);
         else if (c == "resident") g_resident = atoi(argv[i++]);
         else if (c == "capture") g_capture = atoi(argv[i++]) ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;
+        else if (c == "history") history = atoi(argv[i++]);
         else if (c == "release") printf("release %d\n", dlk_release_stream((hipStream_t)strtoull(argv[i++], 0, 0)));
         else {
             dlk_batch b;
@@ -94,6 +97,10 @@ int main(int argc, char **argv) {
             p.temperature = strtof(argv[i + 4], 0);
             p.top_p = 0.9f;
             p.repeat_penalty = 1.0f;
+            if (history) {
+                b.hist_off = b.hist_ids = (const int32_t *)0x40000000ull;
+                p.max_history = history;
+            }
             const hipStream_t s = (hipStream_t)strtoull(argv[i + 5], 0, 0);
             i += 6;
             printf("status %d\n", dlk_sample(&b, rows, vocab, &p, s));

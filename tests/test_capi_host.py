@@ -41,3 +41,20 @@ def test_fresh_workspace_is_cleared_on_the_stream_of_the_call(host, call, kernel
     assert out[0].startswith("malloc") and out[1] == "clear on stream 7" and at[0] == 2, out
     assert not any("memset" in line for line in out), out
     assert sum("clear" in line for line in out) == 1, out       # the kernels return their counters to zero
+
+
+@pytest.mark.parametrize("call,history,kernel", [
+    # greedy over short rows, of any alignment
+    ("1 1001 1001 0 0", 0, "row"), ("64 8193 8193 0 0", 0, "row"), ("64 12288 12288 0 0", 0, "row"),
+    ("64 12292 12292 0 0", 0, "top-k"), ("300 1001 1001 0 0", 0, "top-k"), ("64 4100 4100 0 0", 128, "row"),
+    ("64 8193 8193 0 0", 128, "top-k"), ("64 4100 4100 0 0", 900, "top-k"),
+    # large k
+    ("64 1001 1001 112 1", 0, "top-k"), ("64 1001 1001 150 1", 0, "row"), ("64 12288 12288 150 1", 0, "top-k"),
+    ("8 50257 50257 150 1", 0, "top-k"), ("8 151937 151937 496 1", 0, "row"), ("300 8193 8193 300 1", 0, "top-k"),
+    ("300 8193 8193 496 1", 0, "row"), ("300 50257 50257 496 1", 0, "top-k"), ("64 8193 8193 300 1", 128, "row"),
+    ("64 12288 12288 300 1", 128, "top-k"), ("600 1001 1001 496 1", 0, "top-k")])
+def test_row_kernel_where_it_is_faster(host, call, history, kernel):
+    """Calls whose rows are short or whose k is large run on the row kernel, as rows of odd length did before."""
+    out = host(f"history {history} sample {call} 7")
+    assert sum(f"{kernel} kernel" in line for line in out) == 1 and sum("kernel" in line for line in out) == 1, out
+    assert out[-1] == "status 0"
