@@ -707,7 +707,7 @@ __global__ __launch_bounds__(kFullThreads) void full_kernel(FullParams f) {
     for (int j4 = 0; j4 < EPT / 4; j4++) {
         const int i0 = s0 + 4 * (t + j4 * T);
         float xs[4] = {raw[j4].x, raw[j4].y, raw[j4].z, raw[j4].w};
-        if (CAP) softcap4(xs, p.cap, f.cap_recip);
+        if (CAP) softcap4<false>(xs, p.cap, f.cap_recip);
         if (!whole && i0 >= s1) xs[0] = xs[1] = xs[2] = xs[3] = -INFINITY;
         if (mk) {
             const uint32_t mw = mwd[j4] >> (i0 & 31);

@@ -608,7 +608,7 @@ __global__ __launch_bounds__(kTopkThreads, 8) void topk_kernel(TopkParams f) {
          * half as many each time where their order is no matter.  Turned about each
          * time, so that a sorted slice does not fill cbuf with its worst first.  (The
          * row fell back to one workgroup's selection over all of it: 300 x 50,257 with
-         * k 200 383 us, 91 so; 2 x 131,776 with k 60 and a cap 1,650 and 26; 64 x
+         * k 200 383 us, 91 so; 2 x 131,776 with k 60 and a cap 1,650 and 28; 64 x
          * 50,257 equal logits with k 40 570 and 85; 32 x 262,144 with k 300 1,446 and
          * 137.)  The first pass has a loop of its own: sharing this one made every
          * call 0.6 us slower. */

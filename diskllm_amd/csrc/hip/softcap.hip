@@ -6,11 +6,15 @@
  * host libm's (tanhf_glibc.h).
  *
  * Elementwise work of 8 bytes per element (read + write) that the general form's
- * 80 vector instructions per element made VALU-bound: 512 x 262,144 took 260-270 us
- * where a copy of that size takes 208.  A group of four whose quotients lie in the
- * common range in every lane takes the branch-free form instead: 207 us.  Rows
- * of any alignment take 16-byte loads and stores (4-byte alignment is enough); a
- * workgroup covers 4 * 256 * kSoftcapVec4 elements of one row.
+ * 80 vector instructions per element and its branches made VALU-bound: at
+ * 512 x 262,144 320 to 540 us over fresh logits, by how wide they lie (a copy of that
+ * size takes 208).  A group of four whose quotients lie in the common range in every
+ * lane takes the branch-free form of some 60 instructions, other groups the wide one
+ * of some 75 (softcap4.h): 189 us at cap 30 and sd 4, 211 at sd 5, 222 to 229 at sd
+ * 10 and 30 and at cap 15 and sd 5 (415, 561 and 417 while one value past the common
+ * range sent its group to the general form).  Rows of any alignment take 16-byte
+ * loads and stores (4-byte alignment is enough); a workgroup covers
+ * 4 * 256 * kSoftcapVec4 elements of one row.
  */
 #include <hip/hip_runtime.h>
 
@@ -37,7 +41,7 @@ __global__ __launch_bounds__(kSoftcapThreads) void softcap_vec_kernel(float *__r
         const int i = base + k * kSoftcapThreads * 4;
         if (i + 3 < vocab) {
             float x[4] = {v[k].x, v[k].y, v[k].z, v[k].w};
-            softcap4(x, cap, recip);
+            softcap4<true>(x, cap, recip);
             store4(row + i, make_float4(x[0], x[1], x[2], x[3]));
         } else {
             for (int c = 0; c < 4 && i + c < vocab; c++) row[i + c] = dlk_softcap_glibc(row[i + c], cap);

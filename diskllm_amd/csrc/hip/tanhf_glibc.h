@@ -197,4 +197,51 @@ DLK_TH float dlk_softcap_common(float x, float q, float cap) {
     return __builtin_copysignf(cap * dlk_div_inner(-y, y + 2.0f), x);
 }
 
+/* ---- and for all but a few values, branch-free ----------------------------------
+ * q in [2^-60, 7.75): expm1f's argument is -2 q below 1 and 2 q from there on, and
+ * k is one of 0, -1, -2, -3 or 3 .. 22, so every per-k form is (A + d) 2^k - B with
+ * d = r - e: A is 1 - 2^-k from k = 3 on, 1 at k = -2 and -3, else 0; B is 1 at
+ * k = -2 and -3, 1/2 at k = -1, else 0 (adding or subtracting 0 and scaling by a
+ * power of two change nothing).  The two special ranges of the reduction give the
+ * same k and the same hi, lo and c as its general form there.  x = 0 comes out as
+ * 0, and from 16 cap on tanhf is 1 (its 1 - 2 / (t + 2) rounds to 1 from q = 9.02). */
+#define DLK_SOFTCAP_WIDE_SPAN (0x40f80000u - 0x21800000u)
+#define DLK_SOFTCAP_ONE 16.0f
+
+/* Whether dlk_softcap_wide holds for x (q = dlk_softcap_quot of it; cap16 = 16 cap). */
+DLK_TH int dlk_softcap_wide_ok(float x, float q, float cap16) {
+    return (dlk_softcap_place(q) < DLK_SOFTCAP_WIDE_SPAN) | (x == 0.0f) | (__builtin_fabsf(x) >= cap16);
+}
+
+/* cap * tanhf(x / cap) where dlk_softcap_wide_ok. */
+DLK_TH float dlk_softcap_wide(float x, float q, float cap, float cap16) {
+    const float kLn2Hi = dlk_th_u2f(0x3f317180u), kLn2Lo = dlk_th_u2f(0x3717f7d1u);
+    const float kInvLn2 = dlk_th_u2f(0x3fb8aa3bu);
+    const float kQ1 = dlk_th_u2f(0xbd088889u), kQ2 = dlk_th_u2f(0x3ad00d01u), kQ3 = dlk_th_u2f(0xb8a670cdu),
+                kQ4 = dlk_th_u2f(0x36867e54u), kQ5 = dlk_th_u2f(0xb457edbbu);
+    const int one = __builtin_fabsf(x) >= cap16;
+    q = one ? 1.0f : q;                                /* (any value of the range) */
+    const int neg = q < 1.0f;
+    const float x2 = neg ? -2.0f * q : 2.0f * q;
+    const int k = (int)(kInvLn2 * x2 + (neg ? -0.5f : 0.5f));
+    const float kf = (float)k;
+    const float hi = x2 - kf * kLn2Hi;
+    const float lo = kf * kLn2Lo;
+    const float r = hi - lo;
+    const float c = (hi - r) - lo;
+    const float hfx = 0.5f * r;
+    const float hxs = r * hfx;
+    const float r1 = 1.0f + hxs * (kQ1 + hxs * (kQ2 + hxs * (kQ3 + hxs * (kQ4 + hxs * kQ5))));
+    const float t = 3.0f - r1 * hfx;
+    float e = hxs * dlk_div_inner(r1 - t, 6.0f - r * t);
+    e = r * (e - c) - c;
+    e -= hxs;
+    const float A = k > 0 ? 1.0f - __builtin_ldexpf(1.0f, -k) : k < -1 ? 1.0f : 0.0f;
+    const float B = k >= 0 ? 0.0f : k == -1 ? 0.5f : 1.0f;
+    const float y = __builtin_ldexpf(A + (r - e), k) - B;
+    const float d = dlk_div_inner(neg ? -y : 2.0f, y + 2.0f);
+    const float z = one ? 1.0f : neg ? d : 1.0f - d;
+    return __builtin_copysignf(cap * z, x);
+}
+
 #endif
