@@ -433,7 +433,7 @@ int launch_full(dlk::RowParams p, int rows, int vocab, int max_hist, int force_e
     for (int r0 = 0; r0 < rows; r0 += rows_per) {
         const int nr = rows - r0 < rows_per ? rows - r0 : rows_per;
         f.p = rows_from(p, r0);
-        f.halves = nr % 8 == 0 && G % 2 == 0 && nr * G <= cap;
+        f.map = full_map(nr, G, cap);
         if (dlk_launch_full_kernel(&f, nr, ept, lds, stream) != 0) return DLK_ERR_HIP;
     }
     return DLK_OK;

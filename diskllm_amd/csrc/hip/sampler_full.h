@@ -5,6 +5,7 @@
 #define DLK_SAMPLER_FULL_H
 
 #include "sampler_params.h"
+#include "sampler_map.h"
 
 namespace dlk {
 
@@ -53,7 +54,7 @@ struct FullParams {
     int S;             /* slice length = EPT * kFullThreads */
     int max_hist;      /* longer histories are flagged (DLK_STATUS_HISTORY_TOO_LONG) */
     float cap_recip;   /* dlk_softcap_recip(p.cap) */
-    int halves;        /* block -> (row, slice): each row's slices from both halves of its XCD's blocks */
+    int map;           /* workgroup -> (row, slice): kMap* */
     int stage_cap;     /* chunks of final probabilities kept in LDS per workgroup */
     uint32_t *sync;    /* [rows][kSyncWords] */
     uint64_t *pub;     /* [rows][G][kPubWords], in the zeroed counter region: a word that readers

@@ -494,35 +494,8 @@ __global__ __launch_bounds__(kFullThreads) void full_kernel(FullParams f) {
     extern __shared__ __align__(16) unsigned char smem[];
     const RowParams &p = f.p;
     const int G = f.G, T = kFullThreads;
-    /* a row's workgroups on one XCD: dispatch deals workgroup b to XCD b % 8,
-     * so for whole groups of eight rows, the rows of b % 8 are those of XCD
-     * b % 8.  With halves (a grid that is resident at once, of whole groups of
-     * eight rows): among an XCD's blocks, the first half are the first
-     * block of their CU and the second half the second (two per CU), and the
-     * second block of a CU runs behind the first (older waves win issue): so a
-     * row takes half its slices from each half, rather than all of a row's
-     * slices running behind.  The first half takes slice 0 (the start of the
-     * draw, the row's longest draw phase) and the last G/2 - 1 slices (where
-     * the top-p crossing of a spread-out row lies, which the others wait for) */
     int row, g;
-    const int rows8 = ((int)gridDim.x / G) & ~7;   /* rows of whole groups of eight */
-    if (f.halves) {
-        /* k: the block's place among its XCD's blocks; the first and second
-         * halves of them are the first and second block of their CUs: each row
-         * takes G/2 slices from each half */
-        const int k = blockIdx.x >> 3, R = (int)(gridDim.x >> 4), h = G >> 1;
-        const int k2 = k < R ? k : k - R;
-        row = (k2 / h) * 8 + (blockIdx.x & 7);
-        const int i = k2 % h;
-        g = k < R ? (i == 0 ? 0 : G - h + i) : 1 + i;
-    } else if ((int)blockIdx.x < rows8 * G) {
-        const int k = blockIdx.x >> 3;
-        row = (k / G) * 8 + (blockIdx.x & 7);
-        g = k % G;
-    } else {
-        row = blockIdx.x / G;
-        g = blockIdx.x % G;
-    }
+    full_place((int)blockIdx.x, (int)gridDim.x, G, f.map, &row, &g);
     const int t = threadIdx.x, lane = lane_id();
     const int V = p.V, S = f.S, nch = S / 64;
     const int s0 = g * S, s1 = min(V, s0 + S);
@@ -1646,14 +1619,8 @@ extern "C" int dlk_launch_full_kernel(const dlk::FullParams *f, int rows, int ep
     }
     /* An ordinary launch (a cooperative one costs ~12 us of launch latency
      * here), of any number of rows: a workgroup waits only on workgroups of its
-     * own row.  With `halves` the host has checked that the whole grid is
-     * resident at once (dlk_full_kernel_capacity).  Otherwise the grid may be
-     * larger: each XCD is dealt its workgroups in index order, and on each XCD
-     * every workgroup of an earlier row (of the XCD's rows, or of all rows where
-     * they are spread) has the lower index, so the workgroups of the first row
-     * that is not finished are always the next to get a place, never behind
-     * those of a later row: it finishes, and by induction so do all.  Every wait
-     * is bounded besides. */
+     * own row, and the mapping that the host chose lets every row finish
+     * (sampler_map.h).  Every wait is bounded besides. */
     FullParams fp = *f;
     void *args[] = {&fp};
     if (hipLaunchKernel(fn, dim3(rows * f->G), dim3(kFullThreads), args, lds, stream) != hipSuccess) return -1;

@@ -65,7 +65,11 @@ static int launched(void) { return hipGetLastError() == hipSuccess ? 0 : -1; }
 int dlk_launch_row_kernel(const dlk::RowParams *, int rows, size_t, hipStream_t s) { printf("row kernel, %d rows on stream %zu\n", rows, (size_t)s); return launched(); }
 int dlk_launch_topk_kernel(const dlk::TopkParams *, int rows, size_t, hipStream_t s) { printf("top-k kernel, %d rows on stream %zu\n", rows, (size_t)s); return launched(); }
 int dlk_topk_kernel_occupancy(int, size_t) { return 4; }
-int dlk_launch_full_kernel(const dlk::FullParams *, int rows, int, size_t, hipStream_t s) { printf("fused kernel, %d rows on stream %zu\n", rows, (size_t)s); return launched(); }
+int dlk_launch_full_kernel(const dlk::FullParams *f, int rows, int, size_t, hipStream_t s) {
+    printf("fused kernel, %d rows on stream %zu\n", rows, (size_t)s);
+    printf("mapping %d\n", f->map);
+    return launched();
+}
 int dlk_full_kernel_capacity(int, size_t, int, int) { return g_resident; }
 int dlk_launch_long_history_penalties(float *, int64_t, int, int, const int32_t *, const int32_t *, uint32_t, float, float, float, int, int32_t *, const uint64_t *, uint64_t *, hipStream_t) { printf("penalties\n"); return launched(); }
 int dlk_launch_long_history_fixup(int, const int32_t *, const uint64_t *, uint64_t *, int32_t *, uint32_t *, hipStream_t) { return launched(); }

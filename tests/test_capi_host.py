@@ -37,6 +37,7 @@ def test_fresh_workspace_is_cleared_on_the_stream_of_the_call(host, call, kernel
     is not waited for by a non-blocking one, and the kernel's row barriers then count from whatever is there."""
     out = host(f"sample {call} 7 sample {call} 7")
     at = [i for i, line in enumerate(out) if "kernel" in line]
+    at = [i for i in at if "mapping" not in out[i]]
     assert len(at) == 2 and all(out[i] == f"{kernel} kernel, 64 rows on stream 7" for i in at), out
     assert out[0].startswith("malloc") and out[1] == "clear on stream 7" and at[0] == 2, out
     assert not any("memset" in line for line in out), out
@@ -58,3 +59,10 @@ def test_row_kernel_where_it_is_faster(host, call, history, kernel):
     out = host(f"history {history} sample {call} 7")
     assert sum(f"{kernel} kernel" in line for line in out) == 1 and sum("kernel" in line for line in out) == 1, out
     assert out[-1] == "status 0"
+
+
+def test_mapping_follows_the_resident_workgroups(host):
+    """Rows eight apart only where eight rows' workgroups fit the device (64 places: one XCD of eight)."""
+    for resident, rows, want in ((512, 64, 2), (512, 67, 1), (512, 300, 1), (64, 300, 1), (64, 40, 0), (64, 5, 0)):
+        out = host(f"resident {resident} sample {rows} 151936 151936 0 1.0 7")
+        assert f"mapping {want}" in out, (resident, rows, out)

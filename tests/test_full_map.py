@@ -1,0 +1,16 @@
+"""The fused kernel's mapping of workgroups to rows and slices: every row of every grid can finish on any number of
+XCDs (a workgroup holds its place while it waits for its row's others)."""
+import os
+import subprocess
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+def test_every_row_finishes():
+    exe = os.path.join(ROOT, "oracle", "_build", "full_map_check")
+    os.makedirs(os.path.dirname(exe), exist_ok=True)
+    subprocess.run(["g++", "-O2", "-std=c++17", "-o", exe, os.path.join(ROOT, "tests", "native", "full_map_check.cpp")], check=True)
+    grids, stuck, pairs, stuck_pairs, wrong = map(int, subprocess.run([exe], capture_output=True, text=True,
+                                                                     timeout=300).stdout.split())
+    assert grids > 1500 and pairs > 50 and wrong == 0
+    assert stuck == 0 and stuck_pairs == 0

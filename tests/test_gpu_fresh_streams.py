@@ -58,3 +58,44 @@ def test_first_tokens_of_fresh_samplers(cuda):
     for s in objects:
         L.sampler_free(s)
     assert max(slow[2:]) < 0.25, slow                        # (the first two load code objects)
+
+
+@pytest.mark.parametrize("shapes", [((96, 151936), (203, 65536)), ((129, 40961), (516, 20480))])
+def test_two_streams_past_the_resident_workgroups(cuda, shapes):
+    """Two grids of more workgroups than the device holds, let go together on two streams: each row's workgroups wait
+    for one another while both grids' take places by turns."""
+    import torch
+    from diskllm_amd import api
+    work = []
+    for rows, V in shapes:
+        rng = np.random.default_rng(rows)
+        w = make(f"two-{rows}", rows, V, seed=rows, logits=rng.normal(0, 2, (rows, V)).astype(np.float32), top_p=0.92)
+        db = api.to_device(w)
+        st = torch.cuda.Stream()
+        api.sample(db, stream=st.cuda_stream)                # its workspace
+        st.synchronize()
+        db.reset_rng()
+        work.append((w, db, st))
+    busy = torch.empty(1 << 28, device="cuda")
+    torch.cuda.synchronize()
+    for i in range(3):
+        print(f"[case] two streams {shapes} {i}", flush=True)
+        gate = torch.cuda.Stream()
+        with torch.cuda.stream(gate):
+            for k in range(4):
+                busy.fill_(k)
+            go = torch.cuda.Event()
+            go.record()
+        for w, db, st in work:
+            db.reset_rng()
+        torch.cuda.current_stream().synchronize()
+        for w, db, st in work:
+            st.wait_event(go)
+            api.sample(db, stream=st.cuda_stream)
+        torch.cuda.synchronize()
+        for w, db, st in work:
+            res = api.results(db)
+            assert res["status"] == 0
+            for r in range(w.rows):
+                o = O.sample_row(O.prepared_row(w, r), int(w.seeds[r]), w.temperature, w.top_k, w.top_p, w.min_p)
+                assert int(res["ids"][r]) == o["token"] and int(res["states"][r]) == o["state"], (w.name, r)
