@@ -100,7 +100,9 @@ constexpr size_t kScratchCtrWords = (size_t)1 << 16;
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 unsigned char *g_scratch_dev[64];     /* per device: the address of its copy */
 bool g_noalloc = false;               /* set (under g_mu) for a dlk_sample_noalloc call */
-int g_ws_err = DLK_ERR_HIP;           /* why the last workspace() failed */
+constexpr int kNoWorkspace = 2;       /* (from workspace() and the launchers) none can be had: no memory, or the
+                                         stream is being captured.  The row kernel, which needs none, serves */
+int g_ws_err = DLK_ERR_HIP;           /* why the last workspace() failed: a status or kNoWorkspace */
 
 __global__ void zero_words_kernel(uint32_t *p, size_t n) {
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
@@ -161,7 +163,7 @@ bool workspace(hipStream_t stream, int kind, size_t counters, size_t data_bytes,
         /* no allocation while the stream is captured: it would end the capture */
         hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
         if (hipStreamIsCapturing(stream, &cs) != hipSuccess) (void)hipGetLastError();
-        else if (cs != hipStreamCaptureStatusNone) return false;
+        else if (cs != hipStreamCaptureStatusNone) { g_ws_err = kNoWorkspace; return false; }
         if (w->ptr) {
             /* the stream's earlier kernels may still use the old buffer */
             if (hipStreamSynchronize(stream) != hipSuccess) return false;
@@ -169,7 +171,12 @@ bool workspace(hipStream_t stream, int kind, size_t counters, size_t data_bytes,
             w->ptr = nullptr;
             w->ctr_cap = w->data_bytes = 0;
         }
-        if (hipMalloc(&w->ptr, cc * 4 + db) != hipSuccess) { w->ptr = nullptr; return false; }
+        if (hipMalloc(&w->ptr, cc * 4 + db) != hipSuccess) {
+            (void)hipGetLastError();               /* (the next launch would report it as its own) */
+            w->ptr = nullptr;
+            g_ws_err = kNoWorkspace;
+            return false;
+        }
         /* cleared in the order of the call's stream: one that does not wait for the
          * null stream would start its kernels beside a hipMemset there (a first
          * call's row barriers then timed out: 0.55 s and invalid ids) */
@@ -181,6 +188,9 @@ bool workspace(hipStream_t stream, int kind, size_t counters, size_t data_bytes,
     out.data = (unsigned char *)w->ptr + w->ctr_cap * 4;
     return true;
 }
+
+/* The status of a call that nothing serves without a workspace. */
+int ws_status() { return g_ws_err == kNoWorkspace ? DLK_ERR_HIP : g_ws_err; }
 
 size_t fixed_lds(const dlk::LdsPlan &pl) {
     return r16(32 * 8) + r16(64 * 8) + r16(16 * 8) + r16(64 * 4) + 4 * r16((size_t)pl.hfix * 4) +
@@ -204,9 +214,8 @@ dlk::RowParams rows_from(const dlk::RowParams &p, int r0) {
     return q;
 }
 
-/* Rows that are not whole 16-byte groups: where no workspace can be had for the
- * fused kernels (the fixed array is too small, or the stream is being captured
- * and holds none yet) they run on the row kernel, which needs none. */
+/* Rows that are not whole 16-byte groups, where the fixed array of the
+ * no-allocation call is too small: they run on the row kernel. */
 bool row_kernel_instead(const dlk::RowParams &p) { return ((uintptr_t)p.logits & 15) != 0 || (p.ld & 3) != 0; }
 
 /* Where the row kernel (1,024 threads to a row) is the faster one for a top-k or
@@ -237,8 +246,9 @@ bool row_kernel_first(const dlk::RowParams &p, int rows, int vocab, int k, int n
     return plain ? k > 400 || vocab < 160 * (k - 75) : vocab < 50 * (k - 120);
 }
 
-/* Single-pass top-k path (sampler_topk.hip): returns DLK_OK, or 1 when the
- * configuration is outside its range (the caller then uses the row kernel). */
+/* Single-pass top-k path (sampler_topk.hip): returns DLK_OK, 1 when the
+ * configuration is outside its range or kNoWorkspace (the caller then uses the row
+ * kernel). */
 int launch_topk(dlk::RowParams &p, int rows, int vocab, hipStream_t stream) {
     using namespace dlk;
     const int T = kTopkThreads;
@@ -315,15 +325,15 @@ int launch_topk(dlk::RowParams &p, int rows, int vocab, hipStream_t stream) {
     size_t n_slot = r16((size_t)rows * G * sizeof(TopkSlot));
     size_t n_cand = (size_t)rows * G * KP * 8;
     WsView ws;
-    if (!workspace(stream, 0, (size_t)rows, n_slot + n_cand, ws)) return row_kernel_instead(p) ? 1 : g_ws_err;
+    if (!workspace(stream, 0, (size_t)rows, n_slot + n_cand, ws)) return g_noalloc && row_kernel_instead(p) ? 1 : g_ws_err;
     f.counters = ws.counters;
     f.slots = (TopkSlot *)ws.data;
     f.cands = (uint64_t *)(ws.data + n_slot);
     return dlk_launch_topk_kernel(&f, rows, lds, stream) == 0 ? DLK_OK : DLK_ERR_HIP;
 }
 
-/* Fused full-vocabulary path (sampler_full.hip): DLK_OK, or 1 when outside its
- * range (the caller then uses the row kernel). */
+/* Fused full-vocabulary path (sampler_full.hip): DLK_OK, 1 when outside its range
+ * or kNoWorkspace (the caller then uses the row kernel). */
 int launch_full(dlk::RowParams p, int rows, int vocab, int max_hist, int force_exact, int no_wait,
                 hipStream_t stream) {
     using namespace dlk;
@@ -417,13 +427,21 @@ int launch_full(dlk::RowParams p, int rows, int vocab, int max_hist, int force_e
     }
     if (rows_per < rows && rows_per > 8) rows_per &= ~7;
     if (rows_per < 1) return g_noalloc && !row_kernel_instead(p) && (vocab & 3) == 0 ? DLK_ERR_UNSUPPORTED : 1;
-    const size_t n_ln = r16((size_t)rows_per * G * kLaneWords * 8);
     WsView ws;
+    size_t n_ln;
     /* the published words live in the zeroed counter region: they are zero
      * between launches (the kernel returns them to zero) */
-    if (!workspace(stream, 0, (size_t)rows_per * kSyncWords + (size_t)rows_per * G * kPubWords * 2,
-                   n_ln + (size_t)rows_per * fb_bytes, ws))
-        return row_kernel_instead(p) || (vocab & 3) != 0 ? 1 : g_ws_err;
+    while (true) {
+        n_ln = r16((size_t)rows_per * G * kLaneWords * 8);
+        if (workspace(stream, 0, (size_t)rows_per * kSyncWords + (size_t)rows_per * G * kPubWords * 2,
+                      n_ln + (size_t)rows_per * fb_bytes, ws))
+            break;
+        if (g_noalloc) return row_kernel_instead(p) || (vocab & 3) != 0 ? 1 : g_ws_err;
+        /* memory is short: launches of half the rows (680 KB a row at 151,936) */
+        if (g_ws_err != kNoWorkspace || rows_per == 1) return g_ws_err;
+        rows_per /= 2;
+        if (rows_per > 8) rows_per &= ~7;
+    }
     f.sync = ws.counters;
     f.pub = (uint64_t *)(ws.counters + (size_t)rows_per * kSyncWords);
     f.lanes = (uint64_t *)ws.data;
@@ -451,7 +469,7 @@ int launch_row_global_topk(dlk::RowParams &p, int rows, hipStream_t stream) {
     if (rows_per < 1) rows_per = 1;
     if (rows_per > rows) rows_per = rows;
     WsView ws;
-    if (!workspace(stream, 0, 0, (size_t)rows_per * per_row, ws)) return g_ws_err;
+    if (!workspace(stream, 0, 0, (size_t)rows_per * per_row, ws)) return ws_status();
     p.gcand = (uint64_t *)ws.data;
     p.gcand_stride = kpad * 2;
     p.gregion = ws.data + (size_t)rows_per * cand_bytes;
@@ -521,7 +539,7 @@ int sample_impl(const dlk_batch *b, int rows, int vocab, const dlk_sample_params
         const int64_t ldp = ((int64_t)vocab + 63) & ~(int64_t)63;
         const size_t prep_b = r16((size_t)rows * ldp * 4), flag_b = r16((size_t)rows * 4);
         WsView ws;
-        if (!workspace(stream, 1, 0, prep_b + flag_b + (size_t)rows * 8, ws)) return g_ws_err;
+        if (!workspace(stream, 1, 0, prep_b + flag_b + (size_t)rows * 8, ws)) return ws_status();
         float *prep = (float *)ws.data;
         int32_t *too_long = (int32_t *)(ws.data + prep_b);
         uint64_t *rng_saved = (uint64_t *)(ws.data + prep_b + flag_b);
@@ -558,18 +576,21 @@ int sample_impl(const dlk_batch *b, int rows, int vocab, const dlk_sample_params
         else region = aggs_bytes(vocab);
     }
     size_t total = fixed + region;
+    bool no_ws = false;
     /* (greedy under a cap: the row kernel, whose argmax is taken on the capped row) */
     if (prm->path == DLK_PATH_AUTO && (p.greedy || p.topk_on) && !p.s_general && !(p.greedy && cap_on)) {
         int rc = launch_topk(p, rows, vocab, stream);
         if (rc <= 0) return rc;
+        no_ws = rc == kNoWorkspace;
     }
     if ((prm->path == DLK_PATH_AUTO || prm->path == DLK_PATH_FULL_EXACT || prm->path == DLK_PATH_FULL_NO_WAIT) &&
         !p.greedy && !p.topk_on) {
         int rc = launch_full(p, rows, vocab, pl.hcap, prm->path == DLK_PATH_FULL_EXACT,
                              prm->path == DLK_PATH_FULL_NO_WAIT, stream);
         if (rc <= 0) return rc;
+        no_ws = rc == kNoWorkspace;
     }
-    if (total > kMaxLds) return DLK_ERR_UNSUPPORTED;
+    if (total > kMaxLds) return no_ws ? DLK_ERR_HIP : DLK_ERR_UNSUPPORTED;
     pl.bytes = (int)total;
     return dlk_launch_row_kernel(&p, rows, total, stream) == 0 ? DLK_OK : DLK_ERR_HIP;
 }

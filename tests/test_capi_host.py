@@ -66,3 +66,29 @@ def test_mapping_follows_the_resident_workgroups(host):
     for resident, rows, want in ((512, 64, 2), (512, 67, 1), (512, 300, 1), (64, 300, 1), (64, 40, 0), (64, 5, 0)):
         out = host(f"resident {resident} sample {rows} 151936 151936 0 1.0 7")
         assert f"mapping {want}" in out, (resident, rows, out)
+
+
+BIG, ODD = "512 151936 151936 0 1.0", "512 151937 151937 0 1.0"
+
+
+@pytest.mark.parametrize("call", [BIG, ODD])
+def test_less_memory_takes_more_launches(host, call):
+    """A workspace that cannot be had for all rows at once is asked for in half the rows, and again: 350 MB for the
+    whole batch, 25 MB and several launches where that is all there is."""
+    out = host(f"sample {call} 7")
+    assert sum("fused kernel" in line for line in out) == 1 and out[-1] == "status 0", out
+    out = host(f"memory 30000000 sample {call} 7 sample {call} 7")
+    rows = [int(line.split()[2]) for line in out if line.startswith("fused kernel")]
+    assert out.count("status 0") == 2 and sum(rows) == 2 * 512 and max(rows) <= 40, out
+    assert not any("row kernel" in line for line in out)
+    # an earlier call's smaller workspace, freed to make room for the larger, does not stop it either
+    out = host(f"memory 30000000 sample 8 151936 151936 0 1.0 7 sample {call} 7 release 7")
+    assert out.count("status 0") == 2 and sum(line.startswith("malloc ") and "failed" not in line for line in out) == \
+        sum(line == "free block" for line in out), out
+
+
+@pytest.mark.parametrize("call", [FULL, TOPK, ODD, "64 128257 128257 40 0.8"])
+def test_no_memory_at_all_is_left_to_the_row_kernel(host, call):
+    """... which needs none, for rows of every layout."""
+    out = host(f"memory 0 sample {call} 7")
+    assert sum("row kernel" in line for line in out) == 1 and out[-1] == "status 0", out
