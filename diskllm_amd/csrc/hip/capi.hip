@@ -68,7 +68,9 @@ double topp_threshold(float tp) {
  * kind): kernels queued on one stream run in order, so they may share it, and
  * calls on different streams never do.  Kind 0 starts with a counter region
  * that is zero between launches (each launch returns its counters to zero),
- * then scratch; kind 1 holds the prepared logits of dlk_sample's pre-pass.
+ * then scratch; kind 1 holds the prepared logits of dlk_sample's pre-pass.  A buffer
+ * that a graph may hold is not freed when a call needs a larger one: it stays, as kind
+ * -1, until the stream is released.
  * g_mu guards the table and is held by each entry point from its first
  * workspace() through its last launch, so no buffer is regrown (freed) between
  * the moment a call takes its pointers and the moment its kernels are queued. */
@@ -79,6 +81,7 @@ struct WsBuf {
     void *ptr;
     size_t ctr_cap;      /* counter words */
     size_t data_bytes;   /* scratch bytes after the counters */
+    bool captured;       /* a call captured into a graph has taken its address */
 };
 std::mutex g_mu;
 std::vector<WsBuf> g_ws;
@@ -151,9 +154,12 @@ bool workspace(hipStream_t stream, int kind, size_t counters, size_t data_bytes,
     for (auto &e : g_ws)
         if (e.dev == dev && e.stream == stream && e.kind == kind) { w = &e; break; }
     if (!w) {
-        g_ws.push_back(WsBuf{dev, stream, kind, nullptr, 0, 0});
+        g_ws.push_back(WsBuf{dev, stream, kind, nullptr, 0, 0, false});
         w = &g_ws.back();
     }
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &cs) != hipSuccess) (void)hipGetLastError();
+    const bool capturing = cs != hipStreamCaptureStatusNone;
     if (w->ctr_cap < counters || w->data_bytes < data_bytes) {
         size_t cc = w->ctr_cap > counters ? w->ctr_cap : counters;
         if (kind == 0 && cc < 4096) cc = 4096;
@@ -161,10 +167,16 @@ bool workspace(hipStream_t stream, int kind, size_t counters, size_t data_bytes,
         size_t db = w->data_bytes > data_bytes ? w->data_bytes : data_bytes;
         if (db < (1u << 20)) db = 1u << 20;
         /* no allocation while the stream is captured: it would end the capture */
-        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing(stream, &cs) != hipSuccess) (void)hipGetLastError();
-        else if (cs != hipStreamCaptureStatusNone) { g_ws_err = kNoWorkspace; return false; }
-        if (w->ptr) {
+        if (capturing) { g_ws_err = kNoWorkspace; return false; }
+        if (w->ptr && w->captured) {
+            const WsBuf kept{dev, stream, -1, w->ptr, w->ctr_cap, w->data_bytes, true};
+            w->ptr = nullptr;
+            w->ctr_cap = w->data_bytes = 0;
+            w->captured = false;
+            const size_t at = (size_t)(w - g_ws.data());
+            g_ws.push_back(kept);
+            w = &g_ws[at];
+        } else if (w->ptr) {
             /* the stream's earlier kernels may still use the old buffer */
             if (hipStreamSynchronize(stream) != hipSuccess) return false;
             (void)hipFree(w->ptr);
@@ -184,6 +196,7 @@ bool workspace(hipStream_t stream, int kind, size_t counters, size_t data_bytes,
         w->ctr_cap = cc;
         w->data_bytes = db;
     }
+    if (capturing) w->captured = true;
     out.counters = (uint32_t *)w->ptr;
     out.data = (unsigned char *)w->ptr + w->ctr_cap * 4;
     return true;

@@ -113,7 +113,18 @@ int dlk_sample(const dlk_batch *batch, int rows, int vocab, const dlk_sample_par
  * device.  Call it before destroying a stream that was passed to dlk_sample; a
  * later call on the stream allocates afresh.  No counterpart in the reference,
  * whose sampler owns a host work buffer freed by sampler_free
- * (src/sampler.c:91-95). */
+ * (src/sampler.c:91-95).
+ *
+ * HIP graphs: nothing is allocated while `stream` is captured, in any capture
+ * mode, so make each call once on that stream before capturing it.  A captured
+ * call that finds no workspace is recorded on the row kernel, which needs none
+ * and is several times slower (histories past 1,024 ids and top_k above 4,096,
+ * which need one, return DLK_ERR_HIP).  A graph uses the workspace its calls were
+ * captured with: its replays and the stream's other calls must not overlap,
+ * and it is not replayed after this call has released the stream.  A later call
+ * that needs a larger workspace leaves the graph's alone.  Where device memory is
+ * short a call takes its rows in several launches, at the last on the row
+ * kernel. */
 int dlk_release_stream(hipStream_t stream);
 
 /* dlk_sample without any allocation.  No counterpart in the reference: it is

@@ -92,3 +92,27 @@ def test_no_memory_at_all_is_left_to_the_row_kernel(host, call):
     """... which needs none, for rows of every layout."""
     out = host(f"memory 0 sample {call} 7")
     assert sum("row kernel" in line for line in out) == 1 and out[-1] == "status 0", out
+
+
+@pytest.mark.parametrize("call,small,kernel", [(FULL, "2 8192 8192 0 1.0", "fused"), (TOPK, "2 8192 8192 40 0.8", "top-k")])
+def test_capture(host, call, small, kernel):
+    """Nothing is allocated while a stream is captured: a call takes the workspace that an earlier one left, in as many
+    launches as fit it, or else the row kernel."""
+    out = host(f"capture 1 sample {call} 7")
+    assert sum("row kernel" in line for line in out) == 1 and out[-1] == "status 0" and len(out) == 2, out
+    out = host(f"sample {call} 7 capture 1 sample {call} 7")
+    assert sum(f"{kernel} kernel, 64 rows" in line for line in out) == 2, out
+    out = host(f"sample {small} 7 capture 1 sample {call} 7")
+    assert not any("under capture" in line for line in out) and out[-1] == "status 0", out
+
+
+@pytest.mark.parametrize("call,small", [(BIG, FULL), (ODD, "64 151937 151937 0 1.0"), ("512 128257 128257 112 1.0", TOPK)])
+def test_captured_workspace_is_kept(host, call, small):
+    """A graph holds the addresses of the workspace its calls were captured with: a later call that needs more leaves
+    that one alone until the stream is released.  (One that no graph holds makes room.)"""
+    out = host(f"sample {small} 7 capture 1 sample {small} 7 capture 0 sample {call} 7")
+    assert sum(line.startswith("malloc ") for line in out) == 2 and not any("free" in line for line in out), out
+    out = host(f"sample {small} 7 capture 1 sample {small} 7 capture 0 sample {call} 7 sample {call} 7 release 7")
+    assert out[-3:] == ["free block", "free block", "release 0"], out
+    out = host(f"sample {small} 7 sample {call} 7")
+    assert sum("free block" in line for line in out) == 1, out
