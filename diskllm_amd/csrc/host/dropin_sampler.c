@@ -165,35 +165,41 @@ static void report_penalty_failure(uint32_t op) {
 }
 
 static void penalty_one(float *logits, int vocab, const int *seen, int n, uint32_t op, float value) {
-    size_t slots = 64;                              /* hash slots: at most half of them used */
-    while (slots < 2 * (size_t)n) slots <<= 1;
+    int bits = 6;                                   /* hash slots: at most half of them used */
+    while ((size_t)1 << bits < 2 * (size_t)n) bits++;
+    const size_t slots = (size_t)1 << bits;
     int32_t *table = calloc(slots, sizeof(int32_t));   /* entry d + 1 of the distinct ids, 0 = free */
-    int32_t *ids = malloc((size_t)n * sizeof(int32_t));
-    dlk_dropin_ctx *c = table && ids ? dlk_dropin_shared_lock() : NULL;
-    int done = 0;
-    if (c) {
-        if (dlk_dropin_reserve_pinned(c, (size_t)n * (sizeof(float) + sizeof(int32_t))) == 0) {
-            float *vals = (float *)c->pin;
-            int32_t *counts = (int32_t *)c->pin + n;
-            int nd = 0;
-            for (int i = 0; i < n; i++) {
-                const int id = seen[i];
-                if (id < 0 || id >= vocab) continue;
-                size_t h = ((uint32_t)id * 0x9E3779B1u) & (slots - 1);
-                while (table[h] && ids[table[h] - 1] != id) h = (h + 1) & (slots - 1);
-                if (table[h]) {
-                    counts[table[h] - 1]++;
-                } else {
-                    ids[nd] = id;
-                    vals[nd] = logits[id];
-                    counts[nd] = 1;
-                    table[h] = ++nd;
-                }
+    int32_t *ids = malloc((size_t)n * 2 * sizeof(int32_t)), *counts = ids ? ids + n : NULL;
+    int done = 0, nd = 0;
+    if (table && ids) {
+        /* the ids in range, each once, and their counts: before the shared context
+         * is taken, so that threads wait for one another's device work alone (and
+         * not at all where there is nothing to apply) */
+        for (int i = 0; i < n; i++) {
+            const int id = seen[i];
+            if (id < 0 || id >= vocab) continue;
+            /* (the product's high bits: its low ones are those of the id) */
+            size_t h = (size_t)(((uint64_t)(uint32_t)id * 0x9E3779B97F4A7C15ull) >> (64 - bits));
+            while (table[h] && ids[table[h] - 1] != id) h = (h + 1) & (slots - 1);
+            if (table[h]) {
+                counts[table[h] - 1]++;
+            } else {
+                ids[nd] = id;
+                counts[nd] = 1;
+                table[h] = ++nd;
             }
-            const int ok = nd == 0 || dlk_launch_compact_penalty(vals, counts, nd, op, value, c->stream) == DLK_OK;
-            if (nd == 0) {
-                done = 1;
-            } else if (hipStreamSynchronize(c->stream) == hipSuccess && ok) {
+        }
+        done = nd == 0;
+    }
+    dlk_dropin_ctx *c = nd > 0 ? dlk_dropin_shared_lock() : NULL;
+    if (c) {
+        if (dlk_dropin_reserve_pinned(c, (size_t)nd * (sizeof(float) + sizeof(int32_t))) == 0) {
+            float *vals = (float *)c->pin;
+            int32_t *pin_counts = (int32_t *)c->pin + nd;
+            for (int d = 0; d < nd; d++) vals[d] = logits[ids[d]];
+            memcpy(pin_counts, counts, (size_t)nd * sizeof(int32_t));
+            const int ok = dlk_launch_compact_penalty(vals, pin_counts, nd, op, value, c->stream) == DLK_OK;
+            if (hipStreamSynchronize(c->stream) == hipSuccess && ok) {
                 for (int d = 0; d < nd; d++) logits[ids[d]] = vals[d];
                 done = 1;
             }
