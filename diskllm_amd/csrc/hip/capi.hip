@@ -409,7 +409,7 @@ int launch_full(dlk::RowParams p, int rows, int vocab, int max_hist, int force_e
     static CapEntry cap_cache[256];       /* fixed, as occ_cache above */
     static int n_cap = 0;
     const int softcap = p.cap > 0.0f ? 1 : 0;
-    const int hp = p.plan.hcap > kFullThreads ? 2 : 1;    /* history ids per thread */
+    const int hp = p.plan.hcap > kFullThreads ? 2 : 1;    /* instance: kFullHistPer history ids per thread, or 1 */
     int dev = 0, cap = -1;
     if (hipGetDevice(&dev) != hipSuccess) return DLK_ERR_HIP;
     for (int i = 0; i < n_cap; i++) {

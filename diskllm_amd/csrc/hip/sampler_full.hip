@@ -1588,7 +1588,7 @@ const void *full_fn_hp(int which) {
         default: return (const void *)full_kernel<48, CAP, false, HP>;
     }
 }
-/* the instance for (elements per thread, soft-cap, history ids per thread) */
+/* the instance for (elements per thread, soft-cap, one history id per thread or kFullHistPer) */
 const void *full_fn(int which, int cap, int hp) {
     constexpr int kH = dlk::kFullHistPer;
     if (cap) return hp > 1 ? full_fn_hp<true, kH>(which) : full_fn_hp<true, 1>(which);

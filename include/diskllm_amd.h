@@ -133,7 +133,9 @@ int dlk_release_stream(hipStream_t stream);
  * and results as dlk_sample; its workspace is a fixed 64 MiB scratch array per
  * device (held until the process ends), whose counter words each call clears
  * with a fill kernel on `stream`.  Every call on a device shares that device's
- * array, so calls that overlap on one device race.  DLK_ERR_UNSUPPORTED when the
+ * array, so calls that overlap on one device race: those over rows of odd length
+ * or alignment too, which ran without the array before the fused kernels took
+ * such rows.  DLK_ERR_UNSUPPORTED when the
  * call needs more than the array holds or a second buffer: max_history > 1024
  * (the penalties then run on a scratch copy of the rows), or a batch whose
  * kernels' workspace exceeds the array (the fused full-vocabulary kernel takes

@@ -67,9 +67,11 @@ def test_full_vocab_ragged_masked_and_capped(cuda, V):
     run(w, 0, 2)
 
 
-@pytest.mark.parametrize("V,rows,hist", [(50257, 3, 512), (50257, 3, 1024), (50257, 3, 1500)])
+@pytest.mark.parametrize("V,rows,hist", [(50257, 3, 512), (50257, 3, 1024), (50257, 3, 1500), (50257, 3, 4097),
+                                         (50257, 40, 1500)])
 def test_full_vocab_ragged_history_sizes(cuda, V, rows, hist):
-    """Histories that fill the launch's threads, two per thread, and the pre-pass, the last entries among them."""
+    """Histories of one id per thread, of the long-history instances (whose table shares LDS up to 1,024 ids), past
+    those and past the grids they take (the pre-pass), the last entries among them."""
     rng = np.random.default_rng(hist)
     w = batch(V, rows, hist, top_p=0.95)
     lists = [np.concatenate([rng.integers(0, V, hist - 3), [V - 1, V - 2, V - 1]]) for _ in range(rows)]
