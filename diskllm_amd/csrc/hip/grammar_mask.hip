@@ -12,6 +12,7 @@
 #include <math.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "grammar_table.h"
 
@@ -19,10 +20,11 @@ namespace dlk {
 
 constexpr int kMaskTokens = 512;     /* a thread per token: 16 mask words, one 64-byte line per row and block */
 constexpr int kMaskRows = 64;        /* rows per block at most (a wave's lanes, a word's bits) */
-/* Rows are split over blocks up to about this many.  16 x 151,936 JSON rows: 13.7 us
- * at 256, 13.9 at 512, 18.3 at 1,024; 65 x 32,003: 12.8, 12.5, 17.3; 1 to 512 rows of
- * 1,000: 8 to 9.7 at 512, up to 13.8 at 1,024 (all 64 rows to a block: 19). */
-constexpr int kMaskBlocks = 512;
+/* Rows are split over blocks up to about this many.  JSON rows, 16 x 32,000: 9.4 us
+ * at 256 and 300, 11.0 at 512; 64 x 50,257: 17.4, 15.8, 16.6; 64 x 151,936: 30.2,
+ * 25.4, 25.4; 1 to 512 rows of 1,000: 8 to 9.7 at 512, up to 13.8 at 1,024 (all 64
+ * rows to a block: 19). */
+constexpr int kMaskBlocks = 300;
 constexpr int kMaskBytes = 8192;     /* token bytes staged per block (the rest is read from memory) */
 
 /* How a row tests a token: its string fits (len <= room), closes no more braces
@@ -90,27 +92,14 @@ __global__ __launch_bounds__(kMaskTokens) void grammar_mask_kernel(const uint32_
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int t0 = blockIdx.x * kMaskTokens, tok = t0 + t;
     const int r0 = blockIdx.y * per, nr = min(per, rows - r0);
+    /* (the rows' states first, so that they come while the bytes are staged) */
+    dlk_grammar_row st = {};
+    if (wave == 0 && lane < nr) st = states[r0 + lane];
     uint32_t b0 = 0, b1 = 0;
     if (tok < V) { b0 = off[tok]; b1 = off[tok + 1]; }
     /* the block's bytes: [lo, lo + n) staged (a token outside is read from memory) */
     const uint32_t lo = off[t0], hi = off[min(t0 + kMaskTokens, V)];
     const int n = hi > lo ? (int)min(hi - lo, (uint32_t)kMaskBytes) : 0;
-    if (wave == 0) {
-        RowTest r = {};
-        if (lane < nr) r = row_test(states[r0 + lane]);
-        if (__ballot((r.bits & kTable) != 0)) {
-            const int id = (int)(r.bits & (kTable | 0xffu << kStateShift));
-            int first = kMaskRows;
-#pragma unroll 1
-            for (int i = nr - 1; i >= 0; i--)
-                if (id == __builtin_amdgcn_readlane(id, i)) first = i;
-            if (r.bits & kTable) r.bits |= (uint32_t)first << kFirstShift;
-        }
-        if (lane < nr) tests[lane] = r;
-        uint32_t any = 0;
-        for (uint32_t bit = kWalk; bit <= kScan; bit <<= 1) any |= __ballot((r.bits & bit) != 0) ? bit : 0u;
-        if (lane == 0) kinds = any;
-    }
     for (int i0 = 0; i0 < n; i0 += 8 * kMaskTokens) {
         uint8_t x[8];
 #pragma unroll
@@ -123,6 +112,22 @@ __global__ __launch_bounds__(kMaskTokens) void grammar_mask_kernel(const uint32_
             const int i = i0 + k * kMaskTokens + t;
             if (i < n) sb[i] = x[k];
         }
+    }
+    if (wave == 0) {
+        RowTest r = {};
+        if (lane < nr) r = row_test(st);
+        if (__ballot((r.bits & kTable) != 0)) {
+            const int id = (int)(r.bits & (kTable | 0xffu << kStateShift));
+            int first = kMaskRows;
+#pragma unroll 1
+            for (int i = nr - 1; i >= 0; i--)
+                if (id == __builtin_amdgcn_readlane(id, i)) first = i;
+            if (r.bits & kTable) r.bits |= (uint32_t)first << kFirstShift;
+        }
+        if (lane < nr) tests[lane] = r;
+        uint32_t any = 0;
+        for (uint32_t bit = kWalk; bit <= kScan; bit <<= 1) any |= __ballot((r.bits & bit) != 0) ? bit : 0u;
+        if (lane == 0) kinds = any;
     }
     __syncthreads();
 
@@ -216,18 +221,23 @@ __global__ __launch_bounds__(kMaskTokens) void grammar_mask_kernel(const uint32_
             if (dlk_scan_ok(&s)) fed |= 1ull << r;
         }
     }
-    for (int r = 0; r < nr; r++) {
-        const RowTest R = tests[r];
-        /* an escaped first quote does not toggle: the other case's walk from there on */
-        const bool in = ((R.bits & kInStr) != 0) != ((R.bits & flip) != 0);
-        bool ok = fit <= R.room && len > 0 && R.n >= (in ? nb1 : nb0) && R.m >= (in ? nk1 : nk0) &&
-                  !((R.bits & kStart) && lead == 2);
-        if (R.bits & (kTable | kScan)) ok = ok && ((fed >> (R.bits & kTable ? R.bits >> kFirstShift : r)) & 1u);
-        if (tok == eos_id) ok = (R.bits & kFinished) != 0;               /* :285-291 */
-        ok = ok && tok < V;
-        const uint64_t bal = __ballot(ok);
-        if (lane == 0) words[r][wave] = bal;
-    }
+    auto test_rows = [&](auto validated) {         /* (a loop without `fed` where no row needs it: 16 rows 1 us) */
+        for (int r = 0; r < nr; r++) {
+            const RowTest R = tests[r];
+            /* an escaped first quote does not toggle: the other case's walk from there on */
+            const bool in = ((R.bits & kInStr) != 0) != ((R.bits & flip) != 0);
+            bool ok = fit <= R.room && len > 0 && R.n >= (in ? nb1 : nb0) && R.m >= (in ? nk1 : nk0) &&
+                      !((R.bits & kStart) && lead == 2);
+            if (validated && (R.bits & (kTable | kScan)))
+                ok = ok && ((fed >> (R.bits & kTable ? R.bits >> kFirstShift : r)) & 1u);
+            if (tok == eos_id) ok = (R.bits & kFinished) != 0;           /* :285-291 */
+            ok = ok && tok < V;
+            const uint64_t bal = __ballot(ok);
+            if (lane == 0) words[r][wave] = bal;
+        }
+    };
+    if (any & (kTable | kScan)) test_rows(std::true_type{});
+    else test_rows(std::false_type{});
     __syncthreads();
     if (logits && tok < V)
         for (int r = 0; r < nr; r++)

@@ -6,14 +6,13 @@ import subprocess
 import pytest
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
-BUILD = os.path.join(ROOT, "oracle", "_build")
 HIP = "/opt/rocm/bin/hipcc"
 
 
 @pytest.fixture(scope="module")
-def host():
-    os.makedirs(BUILD, exist_ok=True)
-    obj, exe = os.path.join(BUILD, "capi_host.o"), os.path.join(BUILD, "capi_host_check")
+def host(tmp_path_factory):
+    build = tmp_path_factory.mktemp("capi_host")
+    obj, exe = str(build / "capi_host.o"), str(build / "capi_host_check")
     inc = "-I" + os.path.join(ROOT, "include")
     subprocess.run([HIP, "--offload-arch=gfx950", "--offload-host-only", "-O1", "-std=c++17", "-fPIC", inc, "-c",
                     os.path.join(ROOT, "diskllm_amd", "csrc", "hip", "capi.hip"), "-o", obj], check=True)

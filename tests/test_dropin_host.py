@@ -8,10 +8,9 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
 @pytest.mark.parametrize("device", ["device", "nodevice"])
-def test_penalty_calls(device):
+def test_penalty_calls(device, tmp_path):
     """Ids that are all out of range need no device, no lock and no message; the others are counted once each."""
-    exe = os.path.join(ROOT, "oracle", "_build", "dropin_host_check")
-    os.makedirs(os.path.dirname(exe), exist_ok=True)
+    exe = str(tmp_path / "dropin_host_check")
     host = os.path.join(ROOT, "diskllm_amd", "csrc", "host")
     subprocess.run(["gcc", "-O2", "-std=gnu11", "-D__HIP_PLATFORM_AMD__", "-I" + os.path.join(ROOT, "include"),
                     "-I/opt/rocm/include", "-o", exe, os.path.join(ROOT, "tests", "native", "dropin_host_check.c"),

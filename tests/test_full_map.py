@@ -6,9 +6,8 @@ import subprocess
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
-def test_every_row_finishes():
-    exe = os.path.join(ROOT, "oracle", "_build", "full_map_check")
-    os.makedirs(os.path.dirname(exe), exist_ok=True)
+def test_every_row_finishes(tmp_path):
+    exe = str(tmp_path / "full_map_check")
     subprocess.run(["g++", "-O2", "-std=c++17", "-o", exe, os.path.join(ROOT, "tests", "native", "full_map_check.cpp")], check=True)
     grids, stuck, pairs, stuck_pairs, wrong = map(int, subprocess.run([exe], capture_output=True, text=True,
                                                                      timeout=300).stdout.split())

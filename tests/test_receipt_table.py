@@ -5,9 +5,8 @@ import subprocess
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
-def test_receipt_table_is_the_scanner():
-    exe = os.path.join(ROOT, "oracle", "_build", "receipt_table_check")
-    os.makedirs(os.path.dirname(exe), exist_ok=True)
+def test_receipt_table_is_the_scanner(tmp_path):
+    exe = str(tmp_path / "receipt_table_check")
     subprocess.run(["g++", "-O2", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-I" + os.path.join(ROOT, "include"),
                     "-I/opt/rocm/include", "-o", exe, os.path.join(ROOT, "tests", "native", "receipt_table_check.cpp")],
                    check=True)
