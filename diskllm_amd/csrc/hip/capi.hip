@@ -318,9 +318,11 @@ int launch_topk(dlk::RowParams &p, int rows, int vocab, hipStream_t stream) {
     int S = slice_of(gmin);
     for (int g = gmax; g >= gmin; g--) {
         const int s = slice_of(g), gr = (vocab + s - 1) / s;
-        /* (greedy: eight one-batch slices on a CU cost more in their tails than four
-         * of two batches: 64 x 128,256 took 20.3 us against 15.5) */
-        const int64_t fit = resident(lds_for(s, gr)) / (p.greedy && s < 2 * unit ? 2 : 1);
+        /* (greedy over long rows: eight one-batch slices on a CU cost more in their
+         * tails than four of two batches: 64 x 128,256 17.4 us against 12.7, 32 x
+         * 262,144 19.7 and 14.0, 100 x 65,536 11.6 and 10.2; up to 32,000 ids fewer
+         * slices cost more: 300 x 16,384 with 128 ids 13.2 against 20.7) */
+        const int64_t fit = resident(lds_for(s, gr)) / (p.greedy && s < 2 * unit && vocab > 40000 ? 2 : 1);
         if ((int64_t)rows * gr <= fit) { S = s; break; }
     }
     const int G = (vocab + S - 1) / S;

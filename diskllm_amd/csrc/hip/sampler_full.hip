@@ -3,7 +3,7 @@
  * top-p on or off): src/sampler.c:136-234 with k = V, bit-exact, one HBM pass.
  *
  * A row is split over G workgroups of 512 threads, two per CU, resident together
- * (see dlk_launch_full_kernel); each keeps its slice in registers.  The
+ * (sampler_map.h); each keeps its slice in registers.  The
  * row is tied together by row barriers through relaxed agent-scope atomics
  * (every shared word is an atomic store/load; each writer waits for its stores
  * before it signals, so no cache-flushing fences are needed on this path; only

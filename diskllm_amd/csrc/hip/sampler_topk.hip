@@ -8,8 +8,9 @@
  * to finish (relaxed agent-scope atomics: no cache flushes, no spin waits) merges
  * the G candidate lists.  Because s = (l - M) * (1/T) is monotone in l but not
  * injective, the merge re-sorts on s and certifies that no unseen element of any
- * slice can tie the k-th s; rows it cannot certify (long runs of equal s) rerun
- * the exact selection over the whole row in the same workgroup.  The merged top-k
+ * slice comes before the k-th entry under (s desc, index asc); rows it cannot
+ * certify (a run of equal s that the lists do not reach the end of) rerun the exact
+ * selection over the whole row in the same workgroup.  The merged top-k
  * then goes through the exact softmax / top-p / draw pipeline.
  *
  * Reference: src/sampler.c:109-134 (top-k order), :136-234 (pipeline),
@@ -262,7 +263,8 @@ __device__ __noinline__ uint64_t rth_entry(const uint64_t *buf, int n, int r, in
  *   - Groups whose maximum reaches the threshold are listed in LDS; afterwards
  *     they are reloaded (from cache) and their entries at or above the final
  *     threshold become the candidates, of which the first KP under (value desc,
- *     index asc) are published.
+ *     index asc) are published.  Of more than cbuf holds, the KP-th of those in it
+ *     is a bound up to which they are collected again.
  *   - Finite counts come from the mask bits; a non-finite raw logit anywhere in
  *     the slice sends it through an exact recount (NaN / +inf make the row
  *     irregular, -inf is not finite).

@@ -63,8 +63,12 @@ void __hipRegisterVar(void **, void *, char *, const char *, int, size_t, int, i
 
 static int launched(void) { return hipGetLastError() == hipSuccess ? 0 : -1; }
 int dlk_launch_row_kernel(const dlk::RowParams *, int rows, size_t, hipStream_t s) { printf("row kernel, %d rows on stream %zu\n", rows, (size_t)s); return launched(); }
-int dlk_launch_topk_kernel(const dlk::TopkParams *, int rows, size_t, hipStream_t s) { printf("top-k kernel, %d rows on stream %zu\n", rows, (size_t)s); return launched(); }
-int dlk_topk_kernel_occupancy(int, size_t) { return 4; }
+int dlk_launch_topk_kernel(const dlk::TopkParams *f, int rows, size_t, hipStream_t s) {
+    printf("top-k kernel, %d rows on stream %zu\n", rows, (size_t)s);
+    printf("slices %d\n", f->G);
+    return launched();
+}
+int dlk_topk_kernel_occupancy(int, size_t) { return 8; }
 int dlk_launch_full_kernel(const dlk::FullParams *f, int rows, int, size_t, hipStream_t s) {
     printf("fused kernel, %d rows on stream %zu\n", rows, (size_t)s);
     printf("mapping %d\n", f->map);

@@ -115,3 +115,10 @@ def test_captured_workspace_is_kept(host, call, small):
     assert out[-3:] == ["free block", "free block", "release 0"], out
     out = host(f"sample {small} 7 sample {call} 7")
     assert sum("free block" in line for line in out) == 1, out
+
+
+def test_greedy_slices(host):
+    """Greedy slices of two batches only for long rows (at eight workgroups per CU)."""
+    for call, want in (("64 128256 128256 0 0", 16), ("32 262144 262144 0 0", 32), ("300 16384 16384 0 0", 4),
+                       ("128 32000 32000 0 0", 8)):
+        assert f"slices {want}" in host(f"history 200 sample {call} 7"), call
