@@ -82,6 +82,7 @@ struct WsBuf {
     size_t ctr_cap;      /* counter words */
     size_t data_bytes;   /* scratch bytes after the counters */
     bool captured;       /* a call captured into a graph has taken its address */
+    bool large;          /* the stream's fused grids are more than kMapSmallGrid workgroups */
 };
 std::mutex g_mu;
 std::vector<WsBuf> g_ws;
@@ -154,7 +155,7 @@ bool workspace(hipStream_t stream, int kind, size_t counters, size_t data_bytes,
     for (auto &e : g_ws)
         if (e.dev == dev && e.stream == stream && e.kind == kind) { w = &e; break; }
     if (!w) {
-        g_ws.push_back(WsBuf{dev, stream, kind, nullptr, 0, 0, false});
+        g_ws.push_back(WsBuf{dev, stream, kind, nullptr, 0, 0, false, false});
         w = &g_ws.back();
     }
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
@@ -169,7 +170,7 @@ bool workspace(hipStream_t stream, int kind, size_t counters, size_t data_bytes,
         /* no allocation while the stream is captured: it would end the capture */
         if (capturing) { g_ws_err = kNoWorkspace; return false; }
         if (w->ptr && w->captured) {
-            const WsBuf kept{dev, stream, -1, w->ptr, w->ctr_cap, w->data_bytes, true};
+            const WsBuf kept{dev, stream, -1, w->ptr, w->ctr_cap, w->data_bytes, true, false};
             w->ptr = nullptr;
             w->ctr_cap = w->data_bytes = 0;
             w->captured = false;
@@ -200,6 +201,21 @@ bool workspace(hipStream_t stream, int kind, size_t counters, size_t data_bytes,
     out.counters = (uint32_t *)w->ptr;
     out.data = (unsigned char *)w->ptr + w->ctr_cap * 4;
     return true;
+}
+
+/* Notes a fused grid of this many workgroups on the stream; whether no other stream
+ * of the device (nor the no-allocation call, where this is none) has large ones. */
+bool grid_alone(int dev, hipStream_t stream, int64_t blocks) {
+    static bool noalloc_large[64];
+    const bool large = blocks > dlk::kMapSmallGrid;
+    bool alone = g_noalloc || !noalloc_large[dev & 63];
+    if (g_noalloc && large) noalloc_large[dev & 63] = true;
+    for (auto &e : g_ws) {
+        if (e.dev != dev || e.kind != 0) continue;
+        if (e.stream != stream) alone = alone && !e.large;
+        else if (!g_noalloc && large) e.large = true;
+    }
+    return alone;
 }
 
 /* The status of a call that nothing serves without a workspace. */
@@ -463,10 +479,11 @@ int launch_full(dlk::RowParams p, int rows, int vocab, int max_hist, int force_e
     f.fb = ws.data + n_ln;
     f.fb_bytes = fb_bytes;
     f.fb_q_off = fb_q_off;
+    const bool alone = grid_alone(dev, stream, (int64_t)rows_per * G);
     for (int r0 = 0; r0 < rows; r0 += rows_per) {
         const int nr = rows - r0 < rows_per ? rows - r0 : rows_per;
         f.p = rows_from(p, r0);
-        f.map = full_map(nr, G, cap);
+        f.map = full_map(nr, G, cap, alone);
         if (dlk_launch_full_kernel(&f, nr, ept, lds, stream) != 0) return DLK_ERR_HIP;
     }
     return DLK_OK;

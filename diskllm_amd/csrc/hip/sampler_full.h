@@ -15,7 +15,7 @@ constexpr int kFullMaxG = 16;        /* workgroups per row */
 constexpr int kPubWords = 16;        /* 64-bit words each workgroup publishes */
 constexpr int kCandSlots = 2;        /* predicted top-p crossing chunks per workgroup */
 constexpr int kSyncWords = 64;       /* per-row synchronisation words */
-constexpr uint32_t kFullSpinLimit = 1u << 22;   /* polls before a cross-workgroup wait gives up: a few seconds */
+constexpr uint32_t kFullSpinLimit = 1u << 22;   /* polls before a cross-workgroup wait gives up: about 0.55 s */
 
 /* per-row sync words (all zero between launches) */
 enum : int {

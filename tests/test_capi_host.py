@@ -122,3 +122,11 @@ def test_greedy_slices(host):
     for call, want in (("64 128256 128256 0 0", 16), ("32 262144 262144 0 0", 32), ("300 16384 16384 0 0", 4),
                        ("128 32000 32000 0 0", 8)):
         assert f"slices {want}" in host(f"history 200 sample {call} 7"), call
+
+
+def test_rows_in_halves_only_for_the_one_stream_of_large_grids(host):
+    """Two grids with a row's workgroups in both halves can each hold half of every row: the mapping is left as soon as
+    another stream has large grids, and comes back when that is released.  Small grids do not matter."""
+    one, a, b = "sample 1 151936 151936 0 1.0", "sample 64 151936 151936 0 1.0 7", "sample 64 151936 151936 0 1.0 8"
+    out = host(f"{one} 9 {a} {one} 9 {a} {b} {a} {b} release 7 {b}")
+    assert [line for line in out if line.startswith("mapping")] == [f"mapping {m}" for m in (1, 2, 1, 2, 1, 1, 1, 2)], out

@@ -65,7 +65,7 @@ def test_two_streams_past_the_resident_workgroups(cuda, shapes):
     """Two grids of more workgroups than the device holds, let go together on two streams: each row's workgroups wait
     for one another while both grids' take places by turns."""
     import torch
-    from diskllm_amd import api
+    from diskllm_amd import _lib, api
     work = []
     for rows, V in shapes:
         rng = np.random.default_rng(rows)
@@ -99,3 +99,44 @@ def test_two_streams_past_the_resident_workgroups(cuda, shapes):
             for r in range(w.rows):
                 o = O.sample_row(O.prepared_row(w, r), int(w.seeds[r]), w.temperature, w.top_k, w.top_p, w.min_p)
                 assert int(res["ids"][r]) == o["token"] and int(res["states"][r]) == o["state"], (w.name, r)
+    for _, _, st in work:
+        _lib.check(_lib.lib().dlk_release_stream(st.cuda_stream), "dlk_release_stream")
+
+
+def test_three_streams_of_resident_grids(cuda):
+    """Three streams that each keep a batch of 64 rows going, every grid as large as the device."""
+    import torch
+    from diskllm_amd import _lib, api
+    rng = np.random.default_rng(12)
+    rows, V = 64, 151936
+    w = make("three", rows, V, seed=12, logits=rng.normal(0, 2, (rows, V)).astype(np.float32), top_p=0.9)
+    want = []
+    for r in range(rows):
+        state, tokens = int(w.seeds[r]), []
+        row = O.prepared_row(w, r)
+        for _ in range(2):
+            o = O.sample_row(row, state, w.temperature, w.top_k, w.top_p, w.min_p)
+            tokens.append(o["token"])
+            state = o["state"]
+        want.append(tokens)
+    work = []
+    for i in range(3):
+        db, st = api.to_device(w), torch.cuda.Stream()
+        torch.cuda.synchronize()
+        api.sample(db, stream=st.cuda_stream)
+        st.synchronize()
+        assert db.out_ids.cpu().tolist() == [t[0] for t in want]
+        work.append((db, st))
+    for step in range(20):
+        print(f"[case] three streams {step}", flush=True)
+        for db, st in work:
+            with torch.cuda.stream(st):
+                db.reset_rng()
+                for _ in range(2):
+                    api.sample(db, stream=st.cuda_stream)
+        torch.cuda.synchronize()
+        for db, _ in work:
+            assert int(db.status.item()) == 0
+            assert db.out_ids.cpu().tolist() == [t[1] for t in want]
+    for _, st in work:
+        _lib.check(_lib.lib().dlk_release_stream(st.cuda_stream), "dlk_release_stream")
