@@ -1,7 +1,7 @@
 /*
  * oracle.c -- CPU restatement of DiskLLM's token-sampling and grammar-mask path.
  *
- * TEST INFRASTRUCTURE ONLY.  This file is the checker: only tests/, the smoke
+ * TEST INFRASTRUCTURE ONLY.  This file is the oracle: only tests/, the smoke
  * check in __graft_entry__.py and the cpu_baseline leg of bench.py load it.  The
  * product (diskllm_amd/) never links, loads or calls anything here.
  *

@@ -1,4 +1,4 @@
-"""ctypes bindings for the checker.  TEST INFRASTRUCTURE ONLY.
+"""ctypes bindings for the oracle.  TEST INFRASTRUCTURE ONLY.
 
 Loads oracle/_build/liboracle.so (the C restatement in oracle.c) and, when built,
 oracle/_ref/libref_{strict,fast}.so (the reference's own src/sampler.c and
