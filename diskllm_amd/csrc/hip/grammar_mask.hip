@@ -11,20 +11,13 @@
 #include <hip/hip_runtime.h>
 #include <math.h>
 
-#include <algorithm>
 #include <type_traits>
 
+#include "grammar_map.h"
 #include "grammar_table.h"
 
 namespace dlk {
 
-constexpr int kMaskTokens = 512;     /* a thread per token: 16 mask words, one 64-byte line per row and block */
-constexpr int kMaskRows = 64;        /* rows per block at most (a wave's lanes, a word's bits) */
-/* Rows are split over blocks up to about this many.  JSON rows, 16 x 32,000: 9.4 us
- * at 256 and 300, 11.0 at 512; 64 x 50,257: 17.4, 15.8, 16.6; 64 x 151,936: 30.2,
- * 25.4, 25.4; 1 to 512 rows of 1,000: 8 to 9.7 at 512, up to 13.8 at 1,024 (all 64
- * rows to a block: 19). */
-constexpr int kMaskBlocks = 300;
 constexpr int kMaskBytes = 8192;     /* token bytes staged per block (the rest is read from memory) */
 
 /* How a row tests a token: its string fits (len <= room), closes no more braces
@@ -77,7 +70,7 @@ __device__ __forceinline__ RowTest row_test(const dlk_grammar_row &st) {
  * counts (38,000 into one cache line) took 433 us at 16 x 151,936 with counts,
  * this form 17, of which the counting kernel is some 3.  Receipt rows, 16 x
  * 151,936 without counts: 44 us so and 112 when a block resumed its rows' scanner
- * one row after another; 12 now where the rows share a state, 20 where all differ
+ * one row after another; 14 now where the rows share a state, 25 where all differ
  * (65 x 1,000: 7.4, 297, 6.6 and 8.7). */
 __global__ __launch_bounds__(kMaskTokens) void grammar_mask_kernel(const uint32_t *__restrict__ off,
                                                                    const uint8_t *__restrict__ bytes, int V,
@@ -302,12 +295,8 @@ extern "C" int dlk_grammar_mask(const uint32_t *off, const uint8_t *bytes, int v
     using namespace dlk;
     if (!off || !bytes || !states || !mask || vocab <= 0 || rows <= 0 || rows > 65535) return DLK_ERR_INVALID;
     if (mask_ld < (vocab + 31) / 32 || (logits && ld < vocab)) return DLK_ERR_INVALID;
-    /* rows per block: as many as leave about kMaskBlocks blocks (each walks its tokens
-     * again for its rows), between one and kMaskRows */
-    const int gx = (vocab + kMaskTokens - 1) / kMaskTokens;
-    int gy = std::max((rows + kMaskRows - 1) / kMaskRows, std::min(rows, (kMaskBlocks + gx - 1) / gx));
-    const int per = (rows + gy - 1) / gy;
-    gy = (rows + per - 1) / per;
+    const int gx = (vocab + kMaskTokens - 1) / kMaskTokens, per = mask_rows_per_block(vocab, rows);
+    const int gy = (rows + per - 1) / per;
     hipLaunchKernelGGL(grammar_mask_kernel, dim3(gx, gy), dim3(kMaskTokens), 0, stream, off, bytes, vocab, states, rows,
                        per, eos_id, mask, mask_ld, logits, ld);
     if (valid)
