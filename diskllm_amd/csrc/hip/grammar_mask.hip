@@ -68,7 +68,7 @@ __device__ __forceinline__ RowTest row_test(const dlk_grammar_row &st) {
  * flight, and a walk takes four bytes per LDS read.  A walk of dependent byte loads
  * from memory per (token, row) and one atomicAdd per wave and row for the
  * counts (38,000 into one cache line) took 433 us at 16 x 151,936 with counts,
- * this form 17, of which the counting kernel is some 3.  Receipt rows, 16 x
+ * this form 15, of which the counting kernel is some 3.  Receipt rows, 16 x
  * 151,936 without counts: 44 us so and 112 when a block resumed its rows' scanner
  * one row after another; 14 now where the rows share a state, 25 where all differ
  * (65 x 1,000: 7.4, 297, 6.6 and 8.7). */
